@@ -554,6 +554,10 @@ static int plane_launch(chs_context* ctx, int n, const StickArgs& sa, size_t csz
   const size_t tab_bytes = (size_t)n * sizeof(int32_t) + extra_bytes;  // act_of (+ twiddles)
   int nrb = (int)((lim - cmp_bytes - tab_bytes) / row_bytes);
   nrb = std::max(1, std::min(nrb, groups) / std::max(1, nrb_div));
+  // no more row buffers than rows: group g < nrb starts on row g (the plane
+  // kernel loads that row's V_eff ahead of its loop), and a 512-thread
+  // workgroup has more groups than a 32- or 36-point plane has rows
+  nrb = std::min(nrb, n);
   out->nrb = nrb;
   out->threads = threads;
   out->lds = cmp_bytes + (size_t)nrb * row_bytes + tab_bytes;

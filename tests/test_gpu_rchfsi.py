@@ -110,9 +110,6 @@ def test_scf_with_residual_refinement_matches_fp64(ctx, npa):
     assert er[2] <= 3 * e64[2] + 1e-6
 
 
-@pytest.mark.skip(reason="the device faulted while this test ran after the rest of the GPU "
-                         "suite (it passed run on its own with this file); the cause is not "
-                         "found, so the test stays off the device until it is")
 def test_kpoint_scf_with_residual_refinement_matches_fp64(ctx):
     """The same on a k-point set: the 8-atom USPP cell on the Gamma-centred
     {0, 1/2}^3 set (8 k-points with uneven plane-wave counts), the complex64
