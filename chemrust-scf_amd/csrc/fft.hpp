@@ -11,6 +11,8 @@
 // S = +1 is the inverse transform e^{+i 2 pi jk/N}, S = -1 the forward
 // e^{-i 2 pi jk/N}; neither is normalised.
 #pragma once
+#include <type_traits>
+
 #include "common.hpp"
 #include "roots.inc"
 
@@ -119,27 +121,37 @@ template <int S, typename T> struct Dft<9, S, T> : DftCT<3, 3, S, T> {};
 template <int S, typename T> struct Dft<12, S, T> : DftCT<4, 3, S, T> {};
 template <int S, typename T> struct Dft<16, S, T> : DftCT<4, 4, S, T> {};
 
-// Factorisation N = N1 * N2 used for each supported line length.
+// Factorisation N = N1 * N2 used for each supported line length, and the
+// layout of a lane group's scratch tile (RowScratch): pitch PA of its [k1][n2]
+// form, pitch PB of its [m2][k1] form and the stride ST between groups, in
+// 8-byte slots. A row's two exchanges cost the LDS cycles noted (ideal: two
+// per access of a wavefront), counted with 32 lanes per cycle over 32 slot-wide
+// bank pairs; the values are the cheapest of a search over PA, PB and ST (the
+// rule PA = N2 + 1, PB = N1 + 1, ST = span + 17, best at 108 points, cost 222
+// cycles at 72 points, 128 at 64, 168 at 96 and 112 at 36).
 template <int N> struct Split;
-#define CHS_SPLIT(N, A, B)            \
-  template <> struct Split<N> {       \
-    static constexpr int N1 = A;      \
-    static constexpr int N2 = B;      \
+#define CHS_SPLIT(N, A, B, PA_, PB_, ST_) \
+  template <> struct Split<N> {           \
+    static constexpr int N1 = A;          \
+    static constexpr int N2 = B;          \
+    static constexpr int PA = PA_;        \
+    static constexpr int PB = PB_;        \
+    static constexpr int ST = ST_;        \
   };
-CHS_SPLIT(8, 2, 4)
-CHS_SPLIT(12, 3, 4)
-CHS_SPLIT(16, 4, 4)
-CHS_SPLIT(18, 2, 9)
-CHS_SPLIT(24, 4, 6)
-CHS_SPLIT(32, 4, 8)
-CHS_SPLIT(36, 4, 9)
-CHS_SPLIT(48, 4, 12)
-CHS_SPLIT(64, 8, 8)
-CHS_SPLIT(72, 8, 9)
-CHS_SPLIT(96, 8, 12)
-CHS_SPLIT(108, 12, 9)
-CHS_SPLIT(128, 8, 16)
-CHS_SPLIT(144, 12, 12)
+CHS_SPLIT(8, 2, 4, 5, 3, 12)      // 24 (ideal 24)
+CHS_SPLIT(12, 3, 4, 5, 3, 20)     // 28 (ideal 28)
+CHS_SPLIT(16, 4, 4, 5, 5, 20)     // 32 (ideal 32)
+CHS_SPLIT(18, 2, 9, 9, 3, 27)     // 48 (ideal 44)
+CHS_SPLIT(24, 4, 6, 11, 5, 70)    // 48 (ideal 40)
+CHS_SPLIT(32, 4, 8, 9, 5, 40)     // 48 (ideal 48)
+CHS_SPLIT(36, 4, 9, 10, 4, 41)    // 60 (ideal 52)
+CHS_SPLIT(48, 4, 12, 13, 9, 108)  // 64 (ideal 64)
+CHS_SPLIT(64, 8, 8, 9, 9, 72)     // 64 (ideal 64)
+CHS_SPLIT(72, 8, 9, 12, 10, 105)  // 84 (ideal 68)
+CHS_SPLIT(96, 8, 12, 15, 9, 140)  // 80 (ideal 80)
+CHS_SPLIT(108, 12, 9, 10, 13, 137)// 126 (ideal 84)
+CHS_SPLIT(128, 8, 16, 17, 9, 144) // 96 (ideal 96)
+CHS_SPLIT(144, 12, 12, 17, 17, 204)// 96 (ideal 96)
 #undef CHS_SPLIT
 
 // Zero window of a plane line. The wave-function sphere on a grid at least
@@ -468,17 +480,70 @@ template <int N, typename T> struct RowPlanLoad {
   }
 };
 
-// Row scratch of row_apply_v, one per lane group, STRIDE elements apart. The
+// Slot of the group scratch and its access: H passes per exchange, pass h
+// moving component h. complex64 moves whole values. complex128 exchanges its
+// real and then its imaginary parts through the same tile of 8-byte slots,
+// which moves the same bytes in the same LDS cycles and halves the scratch:
+// the scratch bounds the row groups of the complex128 plane kernel (16-byte
+// slots leave 29 groups per CU beside the 98 KB plane of a 108-point grid, one
+// wavefront per SIMD; 8-byte slots 59). The radix-12 and radix-16 second
+// stages (48, 96, 128 and 144 points) keep whole complex128 values: split, the
+// compiler orders their codelets' sums differently in the last bit, and the
+// eigenvectors Rayleigh-Ritz makes of H|psi> may then change sign.
+template <int N, typename T> struct Slot {
+  static constexpr bool WHOLE = sizeof(T) == 4 || Split<N>::N2 > 9;
+  using type = std::conditional_t<WHOLE, cplx<T>, T>;
+  static constexpr int H = WHOLE ? 1 : 2;
+  static __device__ __forceinline__ type put(cplx<T> v, int h) {
+    if constexpr (WHOLE)
+      return v;
+    else
+      return h ? v.y : v.x;
+  }
+  static __device__ __forceinline__ void get(cplx<T>& d, type s, int h) {
+    if constexpr (WHOLE) {
+      d = s;
+    } else {
+      if (h) d.y = s;
+      else d.x = s;
+    }
+  }
+};
+template <int N, typename T> using slot_t = typename Slot<N, T>::type;
+
+// Row scratch of row_apply_v, one per lane group, STRIDE slots apart. The
 // first exchange uses it as [k1][n2] with row pitch PA, the second as
-// [m2][k1] with pitch PB; the pitches and the group stride spread the four
-// exchange patterns of the groups of a wavefront over the LDS banks.
+// [m2][k1] with pitch PB; the pitches and the group stride (Split<N>, for
+// 8-byte slots) spread the four exchange patterns of the groups of a
+// wavefront over the LDS banks.
 template <int N, typename T> struct RowScratch {
   static constexpr int N1 = Split<N>::N1, N2 = Split<N>::N2;
-  static constexpr int PA = sizeof(T) == 4 ? N2 + 1 : N2;
-  static constexpr int PB = N1 + 1;
+  static constexpr bool S8 = sizeof(slot_t<N, T>) == 8;
+  static constexpr int PA = S8 ? Split<N>::PA : N2;
+  static constexpr int PB = S8 ? Split<N>::PB : N1 + 1;
   static constexpr int SPAN = N1 * PA > N2 * PB ? N1 * PA : N2 * PB;
-  static constexpr int STRIDE = SPAN + (sizeof(T) == 4 ? 17 : 20);
+  static constexpr int STRIDE = S8 ? Split<N>::ST : SPAN + 20;
+  static constexpr int BYTES = (int)sizeof(slot_t<N, T>) * STRIDE;
+  static_assert(STRIDE >= SPAN && PA >= N2 && PB >= N1, "tile layout");
 };
+
+// The 3 x 3 tail's exchange through the group scratch (Mid9Tail): lane
+// (t, x) hands y[c] to lane (t, c). Ends with every read issued.
+template <int N, int E, typename T>
+__device__ __forceinline__ void tail_exchange(slot_t<N, T>* sc, cplx<T>* y, int t, int j) {
+  using MT = Mid9Tail<N, T>;
+  using SL = Slot<N, T>;
+  const cplx<T> v[3] = {y[0], y[1], y[2]};
+#pragma unroll
+  for (int h = 0; h < SL::H; ++h) {
+    if (h) wave_sync();
+#pragma unroll
+    for (int c = 0; c < 3; ++c) sc[E + MT::at(t, j, c)] = SL::put(v[c], h);
+    wave_sync();
+#pragma unroll
+    for (int c = 0; c < 3; ++c) SL::get(y[c], sc[E + MT::at(t, c, j)], h);
+  }
+}
 
 // One line of a plane (element j at line[j ES], ES compile-time) by the N2
 // lanes of a group, exchanging through the group's scratch tile sc (the row
@@ -487,51 +552,68 @@ template <int N, typename T> struct RowScratch {
 // LDS bank pair up to four times per 32 lanes. ZIN: the zero window's inputs
 // are not read; ZOUT: its outputs are not stored (Window<N>).
 template <int N, int S, int ES, bool ZIN, bool ZOUT, typename T>
-__device__ __forceinline__ void group_fft_line_x(cplx<T>* line, cplx<T>* sc, int lane,
+__device__ __forceinline__ void group_fft_line_x(cplx<T>* line, slot_t<N, T>* sc, int lane,
                                                  const cplx<T>* __restrict__ tw) {
   constexpr int N1 = Split<N>::N1, N2 = Split<N>::N2;
-  constexpr int R = (N1 + N2 - 1) / N2, PA = RowScratch<N, T>::PA;
+  constexpr int PA = RowScratch<N, T>::PA;
   using W = Window<N>;
-  {
-    cplx<T> a[N1];
-#pragma unroll
-    for (int n1 = 0; n1 < N1; ++n1)
-      a[n1] = ZIN && W::zero_in(n1) ? mk((T)0, (T)0) : line[(n1 * N2 + lane) * ES];
-    Dft<N1, S, T>::run(a);
-#pragma unroll
-    for (int k1 = 1; k1 < N1; ++k1) a[k1] = a[k1] * twiddle<S>(tw, lane * k1);
-#pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) sc[k1 * PA + lane] = a[k1];
-  }
-  wave_sync();
   using MT = Mid9Tail<N, T>;
+  using SL = Slot<N, T>;
+  cplx<T> a[N1];
+#pragma unroll
+  for (int n1 = 0; n1 < N1; ++n1)
+    a[n1] = ZIN && W::zero_in(n1) ? mk((T)0, (T)0) : line[(n1 * N2 + lane) * ES];
+  Dft<N1, S, T>::run(a);
+#pragma unroll
+  for (int k1 = 1; k1 < N1; ++k1) a[k1] = a[k1] * twiddle<S>(tw, lane * k1);
+  // complex128 reads every round's rows (and the tail's) pass by pass, since
+  // its second pass overwrites the tile; complex64 reads them as it goes
+  cplx<T> b[MT::RR][N2], y[3];
+  const int t = lane / 3, j = lane - 3 * t;
+#pragma unroll
+  for (int h = 0; h < SL::H; ++h) {
+    if (h) wave_sync();
+#pragma unroll
+    for (int k1 = 0; k1 < N1; ++k1) sc[k1 * PA + lane] = SL::put(a[k1], h);
+    wave_sync();
+    if constexpr (SL::H > 1) {
+#pragma unroll
+      for (int r = 0; r < MT::RR; ++r)
+        if (lane + r * N2 < N1) {
+#pragma unroll
+          for (int n2 = 0; n2 < N2; ++n2) SL::get(b[r][n2], sc[(lane + r * N2) * PA + n2], h);
+        }
+      if constexpr (MT::on) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) SL::get(y[q], sc[(N2 + t) * PA + 3 * q + j], h);
+      }
+    }
+  }
 #pragma unroll
   for (int r = 0; r < MT::RR; ++r) {
     const int k1 = lane + r * N2;
     if (k1 < N1) {
-      cplx<T> b[N2];
+      if constexpr (SL::H == 1) {
 #pragma unroll
-      for (int n2 = 0; n2 < N2; ++n2) b[n2] = sc[k1 * PA + n2];
-      Dft<N2, S, T>::run(b);
+        for (int n2 = 0; n2 < N2; ++n2) SL::get(b[r][n2], sc[k1 * PA + n2], 0);
+      }
+      Dft<N2, S, T>::run(b[r]);
 #pragma unroll
       for (int k2 = 0; k2 < N2; ++k2)
-        if (!(ZOUT && W::skip_out(k2))) line[(k1 + N1 * k2) * ES] = b[k2];
+        if (!(ZOUT && W::skip_out(k2))) line[(k1 + N1 * k2) * ES] = b[r][k2];
     }
   }
   if constexpr (MT::on) {  // rows k1 = 9 + t by lanes 3 t + j (Mid9Tail)
-    const int t = lane / 3, j = lane - 3 * t, k1 = N2 + t;
-    cplx<T> y[3];
+    const int k1 = N2 + t;
+    if constexpr (SL::H == 1) {
 #pragma unroll
-    for (int a = 0; a < 3; ++a) y[a] = sc[k1 * PA + 3 * a + j];
+      for (int q = 0; q < 3; ++q) SL::get(y[q], sc[k1 * PA + 3 * q + j], 0);
+    }
     Dft<3, S, T>::run(y);
     y[1] = y[1] * twiddle<S>(tw, (N / 9) * j);
     y[2] = y[2] * twiddle<S>(tw, (N / 9) * 2 * j);
     wave_sync();  // every read of the [k1][n2] tile precedes the exchange writes
-#pragma unroll
-    for (int c = 0; c < 3; ++c) sc[MT::E1 + MT::at(t, j, c)] = y[c];
-    wave_sync();
-#pragma unroll
-    for (int bb = 0; bb < 3; ++bb) y[bb] = sc[MT::E1 + MT::at(t, bb, j)];
+    tail_exchange<N, MT::E1>(sc, y, t, j);
     Dft<3, S, T>::run(y);  // X[k2 = j + 3 d]
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -579,12 +661,18 @@ template <int N, typename T> struct RowV {
 // row and the start of the next; otherwise V_eff is read from vrow at the
 // multiply.
 template <int N, typename T, bool PR, bool PF, typename Plan>
-__device__ __forceinline__ void row_apply_v(cplx<T>* crow, cplx<T>* sc, const Plan& rp,
+__device__ __forceinline__ void row_apply_v(cplx<T>* crow, slot_t<N, T>* sc, const Plan& rp,
                                             RowV<N, T>& vv, const T* __restrict__ vrow,
                                             const T* __restrict__ next_vrow, int lane) {
   constexpr int N1 = Split<N>::N1, N2 = Split<N>::N2;
-  constexpr int R = (N1 + N2 - 1) / N2;
+  constexpr int PA = RowScratch<N, T>::PA, PB = RowScratch<N, T>::PB;
   using W = Window<N>;
+  using MT = Mid9Tail<N, T>;
+  using SL = Slot<N, T>;
+  constexpr int RR = MT::RR;
+  cplx<T> b[RR][N2];
+  cplx<T> y[3];  // Mid9Tail: rows k1 = 9 + t by lanes 3 t + j; ends as Z[m2 = j + 3 q]
+  const int tt = lane / 3, tj = lane - 3 * tt, tk1 = N2 + tt;
   {
     cplx<T> a[N1];
 #pragma unroll
@@ -599,19 +687,35 @@ __device__ __forceinline__ void row_apply_v(cplx<T>* crow, cplx<T>* sc, const Pl
     Dft<N1, 1, T>::run(a);
 #pragma unroll
     for (int k1 = 1; k1 < N1; ++k1) a[k1] = a[k1] * rp.w1(k1);
+    // (complex128: both passes' reads here, as in group_fft_line_x)
 #pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) sc[k1 * RowScratch<N, T>::PA + lane] = a[k1];
+    for (int h = 0; h < SL::H; ++h) {
+      if (h) wave_sync();
+#pragma unroll
+      for (int k1 = 0; k1 < N1; ++k1) sc[k1 * PA + lane] = SL::put(a[k1], h);
+      wave_sync();
+      if constexpr (SL::H > 1) {
+#pragma unroll
+        for (int r = 0; r < RR; ++r)
+          if (lane + r * N2 < N1) {
+#pragma unroll
+            for (int n2 = 0; n2 < N2; ++n2) SL::get(b[r][n2], sc[(lane + r * N2) * PA + n2], h);
+          }
+        if constexpr (MT::on) {
+#pragma unroll
+          for (int q = 0; q < 3; ++q) SL::get(y[q], sc[tk1 * PA + 3 * q + tj], h);
+        }
+      }
+    }
   }
-  wave_sync();
-  using MT = Mid9Tail<N, T>;
-  constexpr int RR = MT::RR;
-  cplx<T> b[RR][N2];
 #pragma unroll
   for (int r = 0; r < RR; ++r) {
     const int k1 = lane + r * N2;
     if (k1 < N1) {
+      if constexpr (SL::H == 1) {
 #pragma unroll
-      for (int n2 = 0; n2 < N2; ++n2) b[r][n2] = sc[k1 * RowScratch<N, T>::PA + n2];
+        for (int n2 = 0; n2 < N2; ++n2) SL::get(b[r][n2], sc[k1 * PA + n2], 0);
+      }
       Dft<N2, 1, T>::run(b[r]);
 #pragma unroll
       for (int k2 = 0; k2 < N2; ++k2) {
@@ -627,24 +731,16 @@ __device__ __forceinline__ void row_apply_v(cplx<T>* crow, cplx<T>* sc, const Pl
       for (int m2 = 1; m2 < N2; ++m2) b[r][m2] = b[r][m2] * rp.w2(r, m2);
     }
   }
-  // Mid9Tail: rows k1 = 9 + t by lanes 3 t + j; y ends as Z[m2 = j + 3 q]
-  cplx<T> y[3];
-  int tk1 = 0, tj = 0;
   if constexpr (MT::on) {
-    const int t = lane / 3, j = lane - 3 * t, k1 = N2 + t;
-    tk1 = k1;
-    tj = j;
+    if constexpr (SL::H == 1) {
 #pragma unroll
-    for (int a = 0; a < 3; ++a) y[a] = sc[k1 * RowScratch<N, T>::PA + 3 * a + j];
+      for (int q = 0; q < 3; ++q) SL::get(y[q], sc[tk1 * PA + 3 * q + tj], 0);
+    }
     Dft<3, 1, T>::run(y);
     y[1] = y[1] * rp.w9(1);
     y[2] = y[2] * rp.w9(2);
     wave_sync();  // every read of the [k1][n2] tile precedes the exchange writes
-#pragma unroll
-    for (int c = 0; c < 3; ++c) sc[MT::E1 + MT::at(t, j, c)] = y[c];
-    wave_sync();
-#pragma unroll
-    for (int bb = 0; bb < 3; ++bb) y[bb] = sc[MT::E1 + MT::at(t, bb, j)];
+    tail_exchange<N, MT::E1>(sc, y, tt, tj);
     Dft<3, 1, T>::run(y);  // X[j + 3 d]
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -652,7 +748,7 @@ __device__ __forceinline__ void row_apply_v(cplx<T>* crow, cplx<T>* sc, const Pl
       if constexpr (PF)
         v = vv.vt[d];
       else
-        v = vrow[k1 + N1 * (j + 3 * d)];
+        v = vrow[tk1 + N1 * (tj + 3 * d)];
       y[d] = mk(y[d].x * v, y[d].y * v);
     }
     // forward 3 x 3 with the roles swapped: DFT_3 over d, w_9^{-j p}, then
@@ -660,42 +756,39 @@ __device__ __forceinline__ void row_apply_v(cplx<T>* crow, cplx<T>* sc, const Pl
     Dft<3, -1, T>::run(y);
     y[1] = y[1] * conj(rp.w9(1));
     y[2] = y[2] * conj(rp.w9(2));
-#pragma unroll
-    for (int p = 0; p < 3; ++p) sc[MT::E2 + MT::at(t, j, p)] = y[p];
-    wave_sync();
-#pragma unroll
-    for (int c = 0; c < 3; ++c) y[c] = sc[MT::E2 + MT::at(t, c, j)];
+    tail_exchange<N, MT::E2>(sc, y, tt, tj);
     Dft<3, -1, T>::run(y);  // Z[j + 3 q]
 #pragma unroll
     for (int q = 0; q < 3; ++q) y[q] = y[q] * rp.wt(q);
   }
-  wave_sync();
+  cplx<T> c[N1];
 #pragma unroll
-  for (int r = 0; r < RR; ++r) {
-    const int k1 = lane + r * N2;
-    if (k1 < N1) {
+  for (int h = 0; h < SL::H; ++h) {
+    wave_sync();
 #pragma unroll
-      for (int m2 = 0; m2 < N2; ++m2) sc[m2 * RowScratch<N, T>::PB + k1] = b[r][m2];
+    for (int r = 0; r < RR; ++r) {
+      const int k1 = lane + r * N2;
+      if (k1 < N1) {
+#pragma unroll
+        for (int m2 = 0; m2 < N2; ++m2) sc[m2 * PB + k1] = SL::put(b[r][m2], h);
+      }
     }
-  }
-  if constexpr (MT::on) {
+    if constexpr (MT::on) {
 #pragma unroll
-    for (int q = 0; q < 3; ++q) sc[(tj + 3 * q) * RowScratch<N, T>::PB + tk1] = y[q];
-  }
-  if constexpr (PF)
-    if (next_vrow) vv.load(next_vrow, lane);
-  wave_sync();
-  {
-    cplx<T> c[N1];
-#pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) c[k1] = sc[lane * RowScratch<N, T>::PB + k1];
-    Dft<N1, -1, T>::run(c);
-#pragma unroll
-    for (int m1 = 0; m1 < N1; ++m1) {
-      if (PR && W::zero_in(m1)) continue;
-      const int ai = rp.out(m1);
-      if (ai >= 0) crow[ai] = c[m1];
+      for (int q = 0; q < 3; ++q) sc[(tj + 3 * q) * PB + tk1] = SL::put(y[q], h);
     }
+    if constexpr (PF)
+      if (h == SL::H - 1 && next_vrow) vv.load(next_vrow, lane);
+    wave_sync();
+#pragma unroll
+    for (int k1 = 0; k1 < N1; ++k1) SL::get(c[k1], sc[lane * PB + k1], h);
+  }
+  Dft<N1, -1, T>::run(c);
+#pragma unroll
+  for (int m1 = 0; m1 < N1; ++m1) {
+    if (PR && W::zero_in(m1)) continue;
+    const int ai = rp.out(m1);
+    if (ai >= 0) crow[ai] = c[m1];
   }
   wave_sync();
 }
@@ -705,11 +798,13 @@ __device__ __forceinline__ void row_apply_v(cplx<T>* crow, cplx<T>* sc, const Pl
 // f |y[x]|^2 to orow[x] in FP64. A row belongs to one group, an x to one
 // lane of it, so the update needs no atomics.
 template <int N, typename T, typename Plan>
-__device__ __forceinline__ void row_density(const cplx<T>* crow, cplx<T>* sc, const Plan& rp,
+__device__ __forceinline__ void row_density(const cplx<T>* crow, slot_t<N, T>* sc, const Plan& rp,
                                             double* __restrict__ orow, double f, int lane) {
   constexpr int N1 = Split<N>::N1, N2 = Split<N>::N2;
   constexpr int R = (N1 + N2 - 1) / N2, PA = RowScratch<N, T>::PA;
   using W = Window<N>;
+  using SL = Slot<N, T>;
+  cplx<T> b[R][N2];
   {
     cplx<T> a[N1];
 #pragma unroll
@@ -725,20 +820,33 @@ __device__ __forceinline__ void row_density(const cplx<T>* crow, cplx<T>* sc, co
 #pragma unroll
     for (int k1 = 1; k1 < N1; ++k1) a[k1] = a[k1] * rp.w1(k1);
 #pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) sc[k1 * PA + lane] = a[k1];
+    for (int h = 0; h < SL::H; ++h) {
+      if (h) wave_sync();
+#pragma unroll
+      for (int k1 = 0; k1 < N1; ++k1) sc[k1 * PA + lane] = SL::put(a[k1], h);
+      wave_sync();
+      if constexpr (SL::H > 1) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (lane + r * N2 < N1) {
+#pragma unroll
+            for (int n2 = 0; n2 < N2; ++n2) SL::get(b[r][n2], sc[(lane + r * N2) * PA + n2], h);
+          }
+      }
+    }
   }
-  wave_sync();
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int k1 = lane + r * N2;
     if (k1 < N1) {
-      cplx<T> b[N2];
+      if constexpr (SL::H == 1) {
 #pragma unroll
-      for (int n2 = 0; n2 < N2; ++n2) b[n2] = sc[k1 * PA + n2];
-      Dft<N2, 1, T>::run(b);
+        for (int n2 = 0; n2 < N2; ++n2) SL::get(b[r][n2], sc[k1 * PA + n2], 0);
+      }
+      Dft<N2, 1, T>::run(b[r]);
 #pragma unroll
       for (int k2 = 0; k2 < N2; ++k2) {
-        const double re = (double)b[k2].x, im = (double)b[k2].y;
+        const double re = (double)b[r][k2].x, im = (double)b[r][k2].y;
         orow[k1 + N1 * k2] += f * (re * re + im * im);
       }
     }

@@ -125,6 +125,11 @@ __device__ __forceinline__ void expand_row(const cplx<T>* cmp_row, cplx<T>* rb, 
 // first nrb groups) without the window's inputs (inverse) or outputs
 // (forward), and the rows skip them too and run in the bank-spreading order
 // Window<N>::row.
+// Bound: LDS cycles and exchange latency (one or two wavefronts per SIMD beside
+// the plane). With 8-byte scratch slots in complex128 and the tile pitches of
+// Split<N> the launch went from 5.84 to 4.95 ms (108 points, 512 bands) and
+// from 0.456 to 0.33 ms (72 points, 160 bands); complex64 at 72 points 0.181
+// to 0.165 ms.
 template <int N, typename T, int TPB, bool PR>
 __global__ void __launch_bounds__(TPB) k_plane(cplx<T>* __restrict__ sbuf, StickArgs st,
                                                const T* __restrict__ veff, int nrb, int n_b,
@@ -138,12 +143,12 @@ __global__ void __launch_bounds__(TPB) k_plane(cplx<T>* __restrict__ sbuf, Stick
   const int z = L / n_b, b = L - z * n_b;
   const int RS = PR ? RSW : st.rs;
   cplx<T>* cmp = reinterpret_cast<cplx<T>*>(smem_raw);
-  cplx<T>* rowbuf = cmp + N * RS;
-  int* act_of = reinterpret_cast<int*>(rowbuf + nrb * RowScratch<N, T>::STRIDE);
-  // LT: the rows use RowPlanLds, whose twiddle table follows act_of (N is even,
-  // so the table starts 8-byte aligned)
+  // LT: the rows use RowPlanLds, whose twiddle table lies between the plane
+  // and the row scratch
   constexpr bool LT = sizeof(T) == 4 && TPB == 512;
-  cplx<T>* twl = reinterpret_cast<cplx<T>*>(act_of + N);
+  cplx<T>* twl = cmp + N * RS;
+  slot_t<N, T>* rowbuf = reinterpret_cast<slot_t<N, T>*>(twl + (LT ? LaneTw<N>::SIZE : 0));
+  int* act_of = reinterpret_cast<int*>(rowbuf + nrb * RowScratch<N, T>::STRIDE);
   cplx<T>* plane = sbuf + ((size_t)b * N + z) * st.ld;
   int lane;
   const int g = Groups<N>::id(&lane), ng = Groups<N>::count();
@@ -154,7 +159,8 @@ __global__ void __launch_bounds__(TPB) k_plane(cplx<T>* __restrict__ sbuf, Stick
   // row before); that holds 12 more registers per lane across the row, which
   // the 256-thread complex64 shape has (two wavefronts per SIMD, 256
   // registers each), the 512-thread one with the LDS twiddle plan, and the
-  // 1024-thread shape and complex128 do not.
+  // 1024-thread shape does not. complex128 gains nothing from it (108 points,
+  // 512 bands: 4.99 ms with, 4.95 without).
   constexpr bool PF = sizeof(T) == 4 && TPB <= 512;
   RowV<N, T> vv;
   if (PF && rows) vv.load(vz + (PR ? W::row(g) : g) * N, lane);
@@ -164,7 +170,7 @@ __global__ void __launch_bounds__(TPB) k_plane(cplx<T>* __restrict__ sbuf, Stick
   __syncthreads();
   for (int s = threadIdx.x; s < st.n_st; s += blockDim.x) cmp[st.iy[s] * RS + st.act[s]] = plane[s];
   __syncthreads();
-  cplx<T>* sc = rowbuf + (g >= 0 ? g : 0) * RowScratch<N, T>::STRIDE;
+  slot_t<N, T>* sc = rowbuf + (g >= 0 && g < nrb ? g : 0) * RowScratch<N, T>::STRIDE;
   if constexpr (PR) {
     if (g >= 0 && g < nrb)
       for (int a = g; a < st.n_act; a += nrb)
@@ -360,7 +366,7 @@ k_density_plane_w(const cplx<T>* __restrict__ sbuf,
   using W = Window<N>;
   constexpr int RS = W::RS;
   cplx<T>* cmp = reinterpret_cast<cplx<T>*>(smem_raw);
-  cplx<T>* rowbuf = cmp + N * RS;
+  slot_t<N, T>* rowbuf = reinterpret_cast<slot_t<N, T>*>(cmp + N * RS);
   int* act_of = reinterpret_cast<int*>(rowbuf + nrb * RowScratch<N, T>::STRIDE);
   const int z = blockIdx.x, c = blockIdx.y;
   const int b0 = c * chunk, b1 = min(n_b, b0 + chunk);
@@ -371,7 +377,7 @@ k_density_plane_w(const cplx<T>* __restrict__ sbuf,
   int lane;
   const int g = Groups<N>::id(&lane);
   const bool grp = g >= 0 && g < nrb;
-  cplx<T>* sc = rowbuf + (grp ? g : 0) * RowScratch<N, T>::STRIDE;
+  slot_t<N, T>* sc = rowbuf + (grp ? g : 0) * RowScratch<N, T>::STRIDE;
   const RowPlanRegs<N, T> rp(act_of, tw, grp ? lane : 0);
   for (int b = b0; b < b1; ++b) {
     const double f = occ[b];
@@ -542,10 +548,9 @@ struct PlaneLaunch {
   int threads = 256;
 };
 static int plane_launch(chs_context* ctx, int n, const StickArgs& sa, size_t csz, int n2,
-                        int nrb_div, int threads, int row_elems, PlaneLaunch* out,
+                        int nrb_div, int threads, size_t row_bytes, PlaneLaunch* out,
                         size_t extra_bytes = 0) {
   const size_t cmp_bytes = (size_t)n * sa.rs * csz;
-  const size_t row_bytes = (size_t)row_elems * csz;
   const int lim = max_lds_per_block(ctx);
   if (cmp_bytes + row_bytes + (size_t)n * sizeof(int32_t) + extra_bytes > (size_t)lim)
     return set_error(ctx, CHS_ERR_FFT, "plane of %d^3 grid does not fit in LDS (%zu > %d bytes)",
@@ -677,7 +682,7 @@ static int vloc_pipeline_t(chs_context* ctx, int precision, const void* psi_v, i
       const size_t lanetw = tn.threads == 512 && sizeof(C) == 8
                                 ? (size_t)LaneTw<NN>::SIZE * sizeof(C) : 0;
       CHS_TRY(plane_launch(ctx, NN, sa, sizeof(C), Split<NN>::N2, tn.nrb_div, tn.threads,
-                           RowScratch<NN, T>::STRIDE, &pl, lanetw));
+                           RowScratch<NN, T>::BYTES, &pl, lanetw));
       hipEvent_t* evp = ms ? ev : nullptr;
       if (tn.sb == 16)
         CHS_TRY((vloc_launch<NN, T, 16>(ctx, sa, pl, n_b, psi, sbuf, veff, tw, H.kin, out, aux0,
@@ -826,7 +831,7 @@ static int density_t(chs_context* ctx, const cplx<T>* psi, int n_b, const double
       PlaneLaunch pl;
       if (sa.win) {
         CHS_TRY(plane_launch(ctx, NN, sa, sizeof(cplx<T>), Split<NN>::N2, div, tpb,
-                             RowScratch<NN, T>::STRIDE, &pl));
+                             RowScratch<NN, T>::BYTES, &pl));
         if (tpb == 512)
           hipLaunchKernelGGL((k_density_plane_w<NN, T, 512>), dim3(NN, n_chunks), dim3(512),
                              pl.lds, ctx->stream, sbuf, sa, docc, nb, chunk, pl.nrb, part, tw);
@@ -834,7 +839,8 @@ static int density_t(chs_context* ctx, const cplx<T>* psi, int n_b, const double
           hipLaunchKernelGGL((k_density_plane_w<NN, T, 256>), dim3(NN, n_chunks), dim3(256),
                              pl.lds, ctx->stream, sbuf, sa, docc, nb, chunk, pl.nrb, part, tw);
       } else if constexpr (sizeof(T) == 8) {
-        CHS_TRY(plane_launch(ctx, NN, sa, sizeof(z64), Split<NN>::N2, div, tpb, NN + 1, &pl));
+        CHS_TRY(plane_launch(ctx, NN, sa, sizeof(z64), Split<NN>::N2, div, tpb,
+                             (NN + 1) * sizeof(z64), &pl));
         if (tpb == 512)
           hipLaunchKernelGGL((k_density_plane<NN, 512>), dim3(NN, n_chunks), dim3(512), pl.lds,
                              ctx->stream, sbuf, sa, docc, nb, chunk, pl.nrb, part, tw);
