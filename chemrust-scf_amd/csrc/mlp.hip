@@ -18,8 +18,8 @@
 // minimised by Adam on FP32 master weights, the forward pass always with
 // the bfloat16-rounded weights.
 //
-// Kernels: k_mlp_pass<0> (forward over band-aligned 32-sample tiles in LDS,
-// per-tile sums), k_mlp_band_sums, k_mlp_pass<1> (forward + backward with
+// Kernels: k_mlp_pass<0> (forward over band-aligned 16-sample tiles, per-tile
+// sums), k_mlp_band_sums, k_mlp_pass<1> (forward + backward with
 // the band coefficients, per-block gradient partials), k_mlp_reduce
 // (fixed-order sums), k_mlp_adam, k_mlp_table (one thread per (band, plane
 // wave) inference), and the training-pair builder.
@@ -44,10 +44,7 @@ constexpr int oW1 = 0, oB1 = oW1 + kH * kIn, oW2 = oB1 + kH, oB2 = oW2 + kH * kH
               oW3 = oB2 + kH, oB3 = oW3 + kH * kH, oW4 = oB3 + kH, oB4 = oW4 + kH,
               kNP = oB4 + 1;  // 8705
 static_assert(kNP == CHS_MLP_PARAMS, "parameter count");
-constexpr int kTS = 32;      // samples per training tile
-constexpr int kTSP = kTS + 4;  // row stride of the [feature][sample] activations
-constexpr int kWP = kH + 1;    // padded row stride of W2, W3 in LDS
-constexpr int kMlpBlocks = 512;
+constexpr int kWP = kH + 1;    // padded row stride of W2, W3 in LDS (k_mlp_table)
 
 __device__ __forceinline__ unsigned short f2bf(float f) {
   unsigned int u = __float_as_uint(f);
@@ -56,10 +53,6 @@ __device__ __forceinline__ unsigned short f2bf(float f) {
 }
 __device__ __forceinline__ float bf2f(unsigned short b) { return __uint_as_float((unsigned int)b << 16); }
 __device__ __forceinline__ float silu(float z) { return z / (1.0f + expf(-z)); }
-__device__ __forceinline__ float dsilu(float z) {
-  const float sg = 1.0f / (1.0f + expf(-z));
-  return sg * (1.0f + z * (1.0f - sg));
-}
 __device__ __forceinline__ float tpa_t(float x) {
   const float x2 = x * x, num = 27.0f + 18.0f * x + 12.0f * x2 + 8.0f * x2 * x;
   return num / (num + 16.0f * x2 * x2);
@@ -95,265 +88,390 @@ __device__ __forceinline__ long long batch_index(long long j, long long off, lon
                      (unsigned long long)n);
 }
 
-// Forward + backward of nb samples over 32-sample tiles; gradient partial of
-// this block to part[blockIdx.x][kNP], loss partial to lpart[blockIdx.x].
-// 128 threads: thread (mb, sb) = (t >> 3, t & 7) owns a 4 x 4 output block
-// of every 64 x 32 layer product; for the weight gradients it owns the
-// 4 x 8 block (j, i) = (4 (t >> 3) + q, 8 (t & 7) + p).
+// ---------------------------------------------------------------------------
+// Forward (+ backward) over band-aligned 16-sample tiles, one wavefront per
+// tile and no workgroup barrier inside the tile loop. Every 64 x 64 product
+// is FP32 matrix-core work (v_mfma_f32_16x16x4_f32: lane l = 16 q + i supplies
+// A[i][q] and B[q][i], and holds D[4 q + v][i]):
+//  - activations: lane (q, i) holds sample i's units 16 m + 4 q + v (m, v < 4).
+//    With the K order (m, v) -> unit 16 m + 4 q + v that is exactly the next
+//    layer's B operand, so a layer hands its result on in registers; the
+//    weights are laid out in LDS as those A fragments (one conflict-free
+//    ds_read_b128 per four k-steps), in both orientations for PASS 1;
+//  - weight gradients contract over the 16 samples: D and the layer's input
+//    pass through the wavefront's LDS tile [sample][unit] to get samples into
+//    K; a wavefront accumulates its tiles in registers (144 for W3, W2 and
+//    [W1 | b1]).
+// The 192 activations of a sample are evaluated once per pass. Bound: the
+// FP32 matrix rate (16.9 kflop per sample in PASS 0, 51 in PASS 1) and the
+// exponentials, which run on the vector unit between the products. Measured
+// at 1.53e6 samples: PASS 0 3.77 -> 0.41 ms, PASS 1 7.85 -> 1.10 ms; the former
+// kernel ran on the vector unit with each activation evaluated by 8 or 16
+// threads inside the product loops, and five barriers per product.
+// ---------------------------------------------------------------------------
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+constexpr int kTS = 16;         // samples per tile
+constexpr int kTP = 80;         // floats per row of the transposition tile
+constexpr int kMlpWaves = 4;    // wavefronts per workgroup
+constexpr int kMlpBlocks0 = 1024, kMlpBlocks1 = 256;  // 4 (PASS 0) or 1 wavefront per SIMD
+
+// h = silu(z), ds = silu'(z) from one sigmoid: 1 / (1 + e^-z) as the hardware
+// reciprocal with one Newton step, and z / (1 + e^-z) from it with a residual
+// step (both round as the division does; without the second step the loss and
+// gradient errors double). The sum is kept finite so that the steps have no
+// inf * 0: below z = -69 the sigmoid is 1e-30.
+__device__ __forceinline__ void silu2(float z, float& h, float& ds) {
+  const float d = fminf(1.0f + expf(-z), 1e30f);
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.0f), r, r);
+  h = z * r;
+  h = fmaf(fmaf(-d, h, z), r, h);
+  ds = fmaf(h, 1.0f - r, r);
+}
+
+// Fragment of a 64 x 64 matrix M for the A operand: entry (mo, mi, lane, v) =
+// M[16 mo + i][16 mi + 4 q + v], M = W (forward) or W^T (backward).
+__device__ __forceinline__ void load_fragments(float* __restrict__ f,
+                                               const unsigned short* __restrict__ w, bool transpose) {
+  for (int t = threadIdx.x; t < kH * kH; t += blockDim.x) {
+    const int v = t & 3, lane = (t >> 2) & 63, mi = (t >> 8) & 3, mo = t >> 10;
+    const int r = 16 * mo + (lane & 15), c = 16 * mi + 4 * (lane >> 4) + v;
+    f[t] = bf2f(transpose ? w[c * kH + r] : w[r * kH + c]);
+  }
+}
+
+// out = M h (+ bias): 64 independent-accumulator MFMAs.
+__device__ __forceinline__ void mlp_product(const f32x4* __restrict__ frag, int lane,
+                                            const float (&h)[4][4], f32x4 (&acc)[4]) {
+#pragma unroll
+  for (int mi = 0; mi < 4; ++mi) {
+    f32x4 a[4];
+#pragma unroll
+    for (int mo = 0; mo < 4; ++mo) a[mo] = frag[(mo * 4 + mi) * 64 + lane];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int mo = 0; mo < 4; ++mo)
+        acc[mo] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[mo][v], h[mi][v], acc[mo], 0, 0, 0);
+  }
+}
+
+// Per-wavefront orderings of its own LDS tile.
+__device__ __forceinline__ void mlp_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Batch: nbb whole bands; batch band j is band (off + j stride) mod NB of
 // the pair arrays (band length Lb); tile tt = (j, q0) covers samples q0 ..
-// q0 + 31 of band j. PASS 0 writes per-tile sums {sum s a, sum s^2 c,
+// q0 + 15 of band j. PASS 0 writes per-tile sums {sum s a, sum s^2 c,
 // sum |e|^2} to tsum; PASS 1 back-propagates dL/do = g1 (g2 s c - a) s with
-// the band coefficients bcoef[j] = {g1, g2}.
+// the band coefficients bcoef[j] = {g1, g2} and leaves the block's gradient
+// partial in part[blockIdx.x][kNP].
 template <int PASS>
-__global__ void __launch_bounds__(128) k_mlp_pass(const unsigned short* __restrict__ wbf,
-                                                  const float* __restrict__ feat,
-                                                  const float* __restrict__ rr,
-                                                  const float* __restrict__ ee,
-                                                  const float* __restrict__ ww, long long NB,
-                                                  int Lb, int nbb, long long off,
-                                                  long long stride, double* __restrict__ tsum,
-                                                  const double* __restrict__ bcoef,
-                                                  float* __restrict__ part) {
-  __shared__ MlpLds L;
-  __shared__ __attribute__((aligned(16))) float Z1[kH * kTSP], Z2[kH * kTSP], Z3[kH * kTSP];
-  __shared__ __attribute__((aligned(16))) float FT[kIn * kTSP];
-  __shared__ float dO[kTS];
-    load_weights(L, wbf);
-  const int t = threadIdx.x, mb = t >> 3, sb = t & 7;
-  float g3[4][8], g2[4][8], g1[2];
-  for (int q = 0; q < 4; ++q)
-    for (int p = 0; p < 8; ++p) g3[q][p] = g2[q][p] = 0.0f;
-  g1[0] = g1[1] = 0.0f;
-  float gb1 = 0, gb2 = 0, gb3 = 0, gw4 = 0, gb4 = 0;
+__global__ void __launch_bounds__(64 * kMlpWaves)
+__attribute__((amdgpu_waves_per_eu(PASS == 0 ? 4 : 1)))
+k_mlp_pass(const unsigned short* __restrict__ wbf, const float* __restrict__ feat,
+           const float* __restrict__ rr, const float* __restrict__ ee, const float* __restrict__ ww,
+           long long NB, int Lb, int nbb, long long off, long long stride,
+           double* __restrict__ tsum, const double* __restrict__ bcoef, float* __restrict__ part) {
+  constexpr int FW = kH * kH;
+  // weight fragments (after the tile loop of PASS 1: the block's gradient sum)
+  __shared__ __attribute__((aligned(16))) float frag[PASS ? 4 * FW : 2 * FW];
+  __shared__ __attribute__((aligned(16))) float bias[3][kH];
+  __shared__ __attribute__((aligned(16))) float w4s[kH];
+  __shared__ __attribute__((aligned(16))) float tile_mem[PASS ? kMlpWaves * 2 * kTS * kTP : 1];
+  static_assert(4 * FW >= kNP, "the gradient sum reuses the fragments");
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, i = lane & 15;
+  load_fragments(frag, wbf + oW2, false);
+  load_fragments(frag + FW, wbf + oW3, false);
+  if (PASS) {
+    load_fragments(frag + 2 * FW, wbf + oW2, true);
+    load_fragments(frag + 3 * FW, wbf + oW3, true);
+  }
+  if (threadIdx.x < kH) {
+    bias[0][threadIdx.x] = bf2f(wbf[oB1 + threadIdx.x]);
+    bias[1][threadIdx.x] = bf2f(wbf[oB2 + threadIdx.x]);
+    bias[2][threadIdx.x] = bf2f(wbf[oB3 + threadIdx.x]);
+    w4s[threadIdx.x] = bf2f(wbf[oW4 + threadIdx.x]);
+  }
+  const float b4 = bf2f(wbf[oB4]);
+  float w1a[4];  // layer 1's A operand: W1[16 m + i][q]
+#pragma unroll
+  for (int m = 0; m < 4; ++m) w1a[m] = bf2f(wbf[oW1 + (16 * m + i) * kIn + q]);
+  __syncthreads();
+  const f32x4* f2 = reinterpret_cast<const f32x4*>(frag);
+  const f32x4* f3 = f2 + FW / 4;
+  const f32x4* t2 = f2 + 2 * (FW / 4);
+  const f32x4* t3 = f2 + 3 * (FW / 4);
+  auto bias4 = [&](const float* b, int m) {
+    return *reinterpret_cast<const f32x4*>(b + 16 * m + 4 * q);
+  };
+  // PASS 1 accumulators: G[j][i] tiles of W3 and W2; [W1 | b1] in columns 0-4
+  f32x4 g3[4][4], g2[4][4], g1[4];
+  float gw4[4][4], gb3[4][4], gb2[4][4], gb4 = 0.0f;
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    g1[m] = f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      g3[m][p] = g2[m][p] = f32x4{0, 0, 0, 0};
+      gw4[m][p] = gb3[m][p] = gb2[m][p] = 0.0f;
+    }
+  }
   const int tpb = (Lb + kTS - 1) / kTS;
   const long long tiles = (long long)nbb * tpb;
-  // out[m][s] = act_in?(sum_k A(k, m) B[k][s]) for the thread's 4 x 4 block
-  auto mm_fwd = [&](const float* W, int ldw, int K, const float* B, bool silu_b, float acc[4][4]) {
-    for (int k = 0; k < K; ++k) {
-      const float4 bv = *reinterpret_cast<const float4*>(B + k * kTSP + 4 * sb);
-      float b4[4] = {bv.x, bv.y, bv.z, bv.w};
-      if (silu_b)
-        for (int p = 0; p < 4; ++p) b4[p] = silu(b4[p]);
+  float* dt = tile_mem + (PASS ? w * 2 * kTS * kTP : 0);  // D as [sample][unit]
+  float* ht = dt + (PASS ? kTS * kTP : 0);                // the layer's input likewise
+  auto to_tile = [&](float* t, const float (&x)[4][4]) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float a = W[(4 * mb + q) * ldw + k];
+    for (int m = 0; m < 4; ++m)
+      *reinterpret_cast<f32x4*>(t + i * kTP + 16 * m + 4 * q) =
+          f32x4{x[m][0], x[m][1], x[m][2], x[m][3]};
+  };
+  // G[mt][nt] += D H^T over the tile's 16 samples
+  auto wgrad = [&](f32x4 (&g)[4][4]) {
 #pragma unroll
-        for (int p = 0; p < 4; ++p) acc[q][p] = fmaf(a, b4[p], acc[q][p]);
+    for (int t = 0; t < 4; ++t) {
+      float a[4], b[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        a[m] = dt[(4 * t + q) * kTP + 16 * m + i];
+        b[m] = ht[(4 * t + q) * kTP + 16 * m + i];
       }
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          g[m][p] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m], b[p], g[m][p], 0, 0, 0);
     }
   };
-  for (long long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    const int jb = (int)(tile / tpb), q0 = (int)(tile % tpb) * kTS;
+  for (long long tile = (long long)blockIdx.x * kMlpWaves + w; tile < tiles;
+       tile += (long long)gridDim.x * kMlpWaves) {
+    // keeps the fragments in LDS: hoisted out of the loop they would take 128
+    // registers per matrix pair and spill
+    asm volatile("" ::: "memory");
+    const int jb = (int)(tile / tpb), q0 = (int)(tile - (long long)jb * tpb) * kTS;
     const long long base = batch_index(jb, off, stride, NB) * Lb;  // first pair of the band
-    __syncthreads();
-    for (int e = t; e < kIn * kTS; e += blockDim.x) {
-      const int s = e / kIn, c = e % kIn;
-      FT[c * kTSP + s] = q0 + s < Lb ? feat[(base + q0 + s) * kIn + c] : 0.0f;
+    const bool in = q0 + i < Lb;
+    const long long sidx = base + q0 + i;
+    const float fq = in ? feat[sidx * kIn + q] : 0.0f;  // feature q of sample i
+    float h1[4][4], h2[4][4], h3[4][4], d1[4][4], d2[4][4], d3[4][4];
+    auto activate = [&](const f32x4 (&z)[4], float (&h)[4][4], float (&d)[4][4]) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) silu2(z[m][v], h[m][v], d[m][v]);
+    };
+    f32x4 z[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      z[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w1a[m], fq, bias4(bias[0], m), 0, 0, 0);
+    activate(z, h1, d1);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) z[m] = bias4(bias[1], m);
+    mlp_product(f2, lane, h1, z);
+    activate(z, h2, d2);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) z[m] = bias4(bias[2], m);
+    mlp_product(f3, lane, h2, z);
+    activate(z, h3, d3);
+    // output: each lane its 16 units, then the four lanes of the sample
+    float o = 0.0f;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const f32x4 w4v = bias4(w4s, m);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) o = fmaf(w4v[v], h3[m][v], o);
     }
-    __syncthreads();
-    // forward: Z1 = W1 F + b1, Z2 = W2 silu(Z1) + b2, Z3 = W3 silu(Z2) + b3
-    {
-      float acc[4][4];
-      for (int q = 0; q < 4; ++q)
-        for (int p = 0; p < 4; ++p) acc[q][p] = L.b1[4 * mb + q];
-      mm_fwd(L.w1, kIn, kIn, FT, false, acc);
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<float4*>(Z1 + (4 * mb + q) * kTSP + 4 * sb) =
-            make_float4(acc[q][0], acc[q][1], acc[q][2], acc[q][3]);
-    }
-    __syncthreads();
-    {
-      float acc[4][4];
-      for (int q = 0; q < 4; ++q)
-        for (int p = 0; p < 4; ++p) acc[q][p] = L.b2[4 * mb + q];
-      mm_fwd(L.w2, kWP, kH, Z1, true, acc);
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<float4*>(Z2 + (4 * mb + q) * kTSP + 4 * sb) =
-            make_float4(acc[q][0], acc[q][1], acc[q][2], acc[q][3]);
-    }
-    __syncthreads();
-    {
-      float acc[4][4];
-      for (int q = 0; q < 4; ++q)
-        for (int p = 0; p < 4; ++p) acc[q][p] = L.b3[4 * mb + q];
-      mm_fwd(L.w3, kWP, kH, Z2, true, acc);
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<float4*>(Z3 + (4 * mb + q) * kTSP + 4 * sb) =
-            make_float4(acc[q][0], acc[q][1], acc[q][2], acc[q][3]);
-    }
-    __syncthreads();
-    // output s, the band sums (PASS 0) or dL/do (PASS 1) per sample
+    o += __shfl_xor(o, 16);
+    o += __shfl_xor(o, 32);
+    o += b4;
+    const float x = __shfl(fq, i), leb = __shfl(fq, 16 + i);
+    float dO = 0.0f;
     double sa = 0.0, sc = 0.0, se = 0.0;
-    if (t < kTS) {
-      float d = 0.0f;
-      const long long i = base + q0 + t;
-      if (q0 + t < Lb && ww[i] > 0.0f) {
-        float o = L.b4;
-        for (int k = 0; k < kH; ++k) o = fmaf(L.w4[k], silu(Z3[k * kTSP + t]), o);
-        const float x = FT[0 * kTSP + t], eb = expf(FT[1 * kTSP + t]);
-        const float s = tpa_t(x) * expf(o) / eb;
-        const float r0 = rr[2 * i], r1 = rr[2 * i + 1], e0 = ee[2 * i], e1 = ee[2 * i + 1];
-        const float a = -(r0 * e0 + r1 * e1), c = r0 * r0 + r1 * r1;
-        if (PASS == 0) {
-          sa = (double)s * a;
-          sc = (double)s * s * c;
-          se = (double)e0 * e0 + (double)e1 * e1;
-        } else {
-          const float g1 = (float)bcoef[2 * jb], g2 = (float)bcoef[2 * jb + 1];
-          d = g1 * (g2 * s * c - a) * s;
-        }
+    if (in && ww[sidx] > 0.0f) {
+      const float s = tpa_t(x) * expf(o) / expf(leb);
+      const float r0 = rr[2 * sidx], r1 = rr[2 * sidx + 1];
+      const float e0 = ee[2 * sidx], e1 = ee[2 * sidx + 1];
+      const float a = -(r0 * e0 + r1 * e1), c = r0 * r0 + r1 * r1;
+      if (PASS == 0) {
+        sa = (double)s * a;
+        sc = (double)s * s * c;
+        se = (double)e0 * e0 + (double)e1 * e1;
+      } else {
+        const float c1 = (float)bcoef[2 * jb], c2 = (float)bcoef[2 * jb + 1];
+        dO = c1 * (c2 * s * c - a) * s;
       }
-      dO[t] = d;
     }
     if (PASS == 0) {
-      for (int o2 = 32; o2 > 0; o2 >>= 1) {
-        sa += __shfl_down(sa, o2);
-        sc += __shfl_down(sc, o2);
-        se += __shfl_down(se, o2);
+#pragma unroll
+      for (int k = 8; k > 0; k >>= 1) {  // the 16 samples (every q holds them)
+        sa += __shfl_xor(sa, k);
+        sc += __shfl_xor(sc, k);
+        se += __shfl_xor(se, k);
       }
-      if (t == 0) {  // samples live in threads 0 .. 31 (wave 0)
+      if (lane == 0) {
         tsum[3 * tile] = sa;
         tsum[3 * tile + 1] = sc;
         tsum[3 * tile + 2] = se;
       }
       continue;
     }
-    __syncthreads();
-    // output layer gradients; dZ3 = dO w4 dsilu(Z3) in place
-    if (t < kH) {
-      float a = 0.0f;
-      for (int s = 0; s < kTS; ++s) a = fmaf(dO[s], silu(Z3[t * kTSP + s]), a);
-      gw4 += a;
-      if (t == 0)
-        for (int s = 0; s < kTS; ++s) gb4 += dO[s];
-    }
-    __syncthreads();
-    for (int e = t; e < kH * kTS; e += blockDim.x) {
-      const int k = e / kTS, s = e % kTS;
-      Z3[k * kTSP + s] = dO[s] * L.w4[k] * dsilu(Z3[k * kTSP + s]);
-    }
-    __syncthreads();
-    // weight gradient G[j][i] += sum_s D[j][s] act(Bin[i][s]) for the 4 x 8 block
-    auto wgrad = [&](const float* D, const float* Bin, bool silu_b, int nin, float g[4][8]) {
-      for (int s = 0; s < kTS; s += 4) {
-        float dv[4][4], bv[8][4];
-        for (int q = 0; q < 4; ++q) {
-          const float4 v = *reinterpret_cast<const float4*>(D + (4 * mb + q) * kTSP + s);
-          dv[q][0] = v.x; dv[q][1] = v.y; dv[q][2] = v.z; dv[q][3] = v.w;
-        }
-        for (int p = 0; p < 8; ++p) {
-          const int i = 8 * sb + p;
-          if (i < nin) {
-            const float4 v = *reinterpret_cast<const float4*>(Bin + i * kTSP + s);
-            bv[p][0] = v.x; bv[p][1] = v.y; bv[p][2] = v.z; bv[p][3] = v.w;
-            if (silu_b)
-              for (int c = 0; c < 4; ++c) bv[p][c] = silu(bv[p][c]);
-          } else {
-            for (int c = 0; c < 4; ++c) bv[p][c] = 0.0f;
-          }
-        }
-        for (int q = 0; q < 4; ++q)
-          for (int p = 0; p < 8; ++p)
-            for (int c = 0; c < 4; ++c) g[q][p] = fmaf(dv[q][c], bv[p][c], g[q][p]);
+    gb4 += dO;
+    // dZ3 = dO w4 silu'(Z3), then back through W3 and W2
+    float dz[4][4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const f32x4 w4v = bias4(w4s, m);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        gw4[m][v] = fmaf(dO, h3[m][v], gw4[m][v]);
+        dz[m][v] = dO * w4v[v] * d3[m][v];
+        gb3[m][v] += dz[m][v];
       }
+    }
+    auto back = [&](const f32x4* fr, const float (&d)[4][4]) {
+      f32x4 acc[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) acc[m] = f32x4{0, 0, 0, 0};
+      mlp_product(fr, lane, dz, acc);
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dz[m][v] = acc[m][v] * d[m][v];
     };
-    // in-place dZ_prev[i][s] = dsilu(Z_prev[i][s]) * sum_j W[j][i] D[j][s]
-    auto back = [&](const float* W, const float* D, float* Zp) {
-      float acc[4][4];
-      for (int q = 0; q < 4; ++q)
-        for (int p = 0; p < 4; ++p) acc[q][p] = 0.0f;
-      for (int j = 0; j < kH; ++j) {
-        const float4 bv = *reinterpret_cast<const float4*>(D + j * kTSP + 4 * sb);
-        const float b4[4] = {bv.x, bv.y, bv.z, bv.w};
-        for (int q = 0; q < 4; ++q) {
-          const float a = W[j * kWP + 4 * mb + q];
-          for (int p = 0; p < 4; ++p) acc[q][p] = fmaf(a, b4[p], acc[q][p]);
-        }
-      }
-      for (int q = 0; q < 4; ++q) {
-        float* z = Zp + (4 * mb + q) * kTSP + 4 * sb;
-        const float4 zv = *reinterpret_cast<const float4*>(z);
-        *reinterpret_cast<float4*>(z) =
-            make_float4(acc[q][0] * dsilu(zv.x), acc[q][1] * dsilu(zv.y), acc[q][2] * dsilu(zv.z),
-                        acc[q][3] * dsilu(zv.w));
-      }
-    };
-    wgrad(Z3, Z2, true, kH, g3);
-    if (t < kH)
-      for (int s = 0; s < kTS; ++s) gb3 += Z3[t * kTSP + s];
-    __syncthreads();
-    back(L.w3, Z3, Z2);  // Z2 <- dZ2
-    __syncthreads();
-    wgrad(Z2, Z1, true, kH, g2);
-    if (t < kH)
-      for (int s = 0; s < kTS; ++s) gb2 += Z2[t * kTSP + s];
-    __syncthreads();
-    back(L.w2, Z2, Z1);  // Z1 <- dZ1
-    __syncthreads();
-    // W1 gradient (64 x 4 entries, 2 per thread) and b1
-    for (int c = 0; c < 2; ++c) {
-      const int idx = 2 * t + c, j = idx / kIn, i = idx % kIn;
-      float a = 0.0f;
-      for (int s = 0; s < kTS; ++s) a = fmaf(Z1[j * kTSP + s], FT[i * kTSP + s], a);
-      g1[c] += a;
+    to_tile(dt, dz);
+    to_tile(ht, h2);
+    mlp_wave_sync();
+    wgrad(g3);
+    back(t3, d2);
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) gb2[m][v] += dz[m][v];
+    mlp_wave_sync();  // the tile's reads precede its next contents
+    to_tile(dt, dz);
+    to_tile(ht, h1);
+    mlp_wave_sync();
+    wgrad(g2);
+    back(t2, d1);
+    mlp_wave_sync();
+    to_tile(dt, dz);
+    ht[i * kTP + q] = fq;
+    mlp_wave_sync();
+    // [W1 | b1]: features in columns 0-3, ones in column 4
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float fv = ht[(4 * t + q) * kTP + (i & 3)];
+      const float b = i < kIn ? fv : (i == kIn ? 1.0f : 0.0f);
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        g1[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(dt[(4 * t + q) * kTP + 16 * m + i], b, g1[m],
+                                                     0, 0, 0);
     }
-    if (t < kH)
-      for (int s = 0; s < kTS; ++s) gb1 += Z1[t * kTSP + s];
+    mlp_wave_sync();
   }
   if (PASS == 0) return;
-  // block partial in the flat parameter layout
-  float* pb = part + (size_t)blockIdx.x * kNP;
-  for (int q = 0; q < 4; ++q)
-    for (int p = 0; p < 8; ++p) {
-      const int j = 4 * mb + q, i = 8 * sb + p;
-      pb[oW3 + j * kH + i] = g3[q][p];
-      pb[oW2 + j * kH + i] = g2[q][p];
-    }
-  pb[oW1 + 2 * t] = g1[0];
-  pb[oW1 + 2 * t + 1] = g1[1];
-  if (t < kH) {
-    pb[oB1 + t] = gb1;
-    pb[oB2 + t] = gb2;
-    pb[oB3 + t] = gb3;
-    pb[oW4 + t] = gw4;
+  // sums over the 16 samples of the per-lane vectors
+#pragma unroll
+  for (int k = 1; k < 16; k <<= 1) {
+    gb4 += __shfl_xor(gb4, k);
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        gw4[m][v] += __shfl_xor(gw4[m][v], k);
+        gb3[m][v] += __shfl_xor(gb3[m][v], k);
+        gb2[m][v] += __shfl_xor(gb2[m][v], k);
+      }
   }
-  if (t == 0) pb[oB4] = gb4;
+  // the wavefronts add their sums in order into LDS, in the parameter layout
+  for (int ww2 = 0; ww2 < kMlpWaves; ++ww2) {
+    __syncthreads();
+    if (w == ww2) {
+      auto put = [&](int p, float val) { frag[p] = ww2 == 0 ? val : frag[p] + val; };
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int j = 16 * m + 4 * q + v;
+#pragma unroll
+          for (int p = 0; p < 4; ++p) {
+            put(oW3 + j * kH + 16 * p + i, g3[m][p][v]);
+            put(oW2 + j * kH + 16 * p + i, g2[m][p][v]);
+          }
+          if (i < kIn) put(oW1 + j * kIn + i, g1[m][v]);
+          if (i == kIn) put(oB1 + j, g1[m][v]);
+          if (i == 0) {
+            put(oB2 + j, gb2[m][v]);
+            put(oB3 + j, gb3[m][v]);
+            put(oW4 + j, gw4[m][v]);
+          }
+        }
+      if (lane == 0) put(oB4, gb4);
+    }
+  }
+  __syncthreads();
+  float* pb = part + (size_t)blockIdx.x * kNP;
+  for (int p = threadIdx.x; p < kNP; p += blockDim.x) pb[p] = frag[p];
 }
 
-// Per batch band: A, B, E from its tiles (fixed order); L_b = 1 - A^2/(B E)
-// for used bands (B, E > 0), 0 otherwise; bcoef = {2A/(B E) / nbb, A/B};
-// lossv[j] = L_b / nbb.
-__global__ void k_mlp_band_sums(const double* __restrict__ tsum, int nbb, int tpb,
-                                double* __restrict__ bcoef, double* __restrict__ lossv) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= nbb) return;
+// Per batch band, one wavefront: A, B, E from its tiles (lanes over strided
+// tiles, fixed-order shuffle sum); L_b = 1 - A^2/(B E) for used bands (B, E >
+// 0), 0 otherwise; bcoef = {2A/(B E) / nbb, A/B}; lossv[j] = L_b / nbb.
+__global__ void __launch_bounds__(64) k_mlp_band_sums(const double* __restrict__ tsum, int nbb,
+                                                      int tpb, double* __restrict__ bcoef,
+                                                      double* __restrict__ lossv) {
+  const int j = blockIdx.x;
   double A = 0, B = 0, E = 0;
-  for (int q = 0; q < tpb; ++q) {
-    const double* p = tsum + 3 * ((size_t)j * tpb + q);
+  for (int t = threadIdx.x; t < tpb; t += 64) {
+    const double* p = tsum + 3 * ((size_t)j * tpb + t);
     A += p[0];
     B += p[1];
     E += p[2];
   }
+  for (int k = 32; k > 0; k >>= 1) {
+    A += __shfl_xor(A, k);
+    B += __shfl_xor(B, k);
+    E += __shfl_xor(E, k);
+  }
+  if (threadIdx.x != 0) return;
   const bool used = B > 0.0 && E > 0.0;
   bcoef[2 * j] = used ? 2.0 * A / (B * E) / nbb : 0.0;
   bcoef[2 * j + 1] = used ? A / B : 0.0;
   lossv[j] = used ? (1.0 - A * A / (B * E)) / nbb : 0.0;
 }
 
-__global__ void k_mlp_reduce(const float* __restrict__ part, int nblk,
-                             const double* __restrict__ lossv, int nl, float* __restrict__ grad,
-                             double* __restrict__ loss) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < kNP) {
-    double s = 0.0;
-    for (int b = 0; b < nblk; ++b) s += part[(size_t)b * kNP + p];
-    grad[p] = (float)s;
+// Gradient from the block partials, 16 parameters per workgroup with 16
+// threads over the blocks of each (a serial sum per parameter took 0.13 ms);
+// the last workgroup adds up the loss. FP64 sums in a fixed order.
+__global__ void __launch_bounds__(256) k_mlp_reduce(const float* __restrict__ part, int nblk,
+                                                    const double* __restrict__ lossv, int nl,
+                                                    float* __restrict__ grad,
+                                                    double* __restrict__ loss) {
+  __shared__ double sh[16][17];
+  const int c = threadIdx.x & 15, r = threadIdx.x >> 4;
+  const int p = blockIdx.x * 16 + c;
+  double s = 0.0;
+  if (p < kNP)
+    for (int b = r; b < nblk; b += 16) s += part[(size_t)b * kNP + p];
+  sh[r][c] = s;
+  __syncthreads();
+  if (threadIdx.x < 16 && p < kNP) {
+    double t = 0.0;
+    for (int k = 0; k < 16; ++k) t += sh[k][c];
+    grad[p] = (float)t;
   }
-  if (p == 0) {
-    double s = 0.0;
-    for (int b = 0; b < nl; ++b) s += lossv[b];
-    *loss = s;
+  if (blockIdx.x == gridDim.x - 1) {
+    __syncthreads();
+    double l = 0.0;
+    for (int b = threadIdx.x; b < nl; b += 256) l += lossv[b];
+    for (int k = 32; k > 0; k >>= 1) l += __shfl_xor(l, k);
+    if ((threadIdx.x & 63) == 0) sh[0][threadIdx.x >> 6] = l;
+    __syncthreads();
+    if (threadIdx.x == 0) *loss = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
   }
 }
 
@@ -543,23 +661,25 @@ static int mlp_batch(chs_context* ctx, chs_mlp* m, const float* feat, const floa
                      long long stride, double* d_loss) {
   const int tpb = (Lb + kTS - 1) / kTS;
   const long long tiles = (long long)nbb * tpb;
-  CHS_TRY(ensure(ctx, m->part, (size_t)kMlpBlocks * kNP * sizeof(float)));
+  CHS_TRY(ensure(ctx, m->part, (size_t)kMlpBlocks1 * kNP * sizeof(float)));
   CHS_TRY(ensure(ctx, m->tsum, (size_t)tiles * 3 * sizeof(double)));
   CHS_TRY(ensure(ctx, m->bcoef, (size_t)nbb * 3 * sizeof(double)));
   double* bcoef = (double*)m->bcoef.p;
   double* lossv = bcoef + 2 * (size_t)nbb;
-  const int nblk = (int)std::min<long long>(kMlpBlocks, std::max<long long>(1, tiles));
+  const long long want = (tiles + kMlpWaves - 1) / kMlpWaves;
+  const int nblk0 = (int)std::min<long long>(kMlpBlocks0, want);
+  const int nblk1 = (int)std::min<long long>(kMlpBlocks1, want);
   const unsigned short* wbf = (const unsigned short*)m->wbf.p;
-  hipLaunchKernelGGL(k_mlp_pass<0>, dim3(nblk), dim3(128), 0, ctx->stream, wbf, feat, r, e, w, NB,
-                     Lb, nbb, off, stride, (double*)m->tsum.p, (const double*)nullptr,
+  hipLaunchKernelGGL(k_mlp_pass<0>, dim3(nblk0), dim3(64 * kMlpWaves), 0, ctx->stream, wbf, feat, r,
+                     e, w, NB, Lb, nbb, off, stride, (double*)m->tsum.p, (const double*)nullptr,
                      (float*)nullptr);
-  hipLaunchKernelGGL(k_mlp_band_sums, dim3(ceil_div(nbb, 256)), dim3(256), 0, ctx->stream,
+  hipLaunchKernelGGL(k_mlp_band_sums, dim3(nbb), dim3(64), 0, ctx->stream,
                      (const double*)m->tsum.p, nbb, tpb, bcoef, lossv);
-  hipLaunchKernelGGL(k_mlp_pass<1>, dim3(nblk), dim3(128), 0, ctx->stream, wbf, feat, r, e, w, NB,
-                     Lb, nbb, off, stride, (double*)nullptr, (const double*)bcoef,
+  hipLaunchKernelGGL(k_mlp_pass<1>, dim3(nblk1), dim3(64 * kMlpWaves), 0, ctx->stream, wbf, feat, r,
+                     e, w, NB, Lb, nbb, off, stride, (double*)nullptr, (const double*)bcoef,
                      (float*)m->part.p);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3(ceil_div(kNP, 256)), dim3(256), 0, ctx->stream,
-                     (const float*)m->part.p, nblk, (const double*)lossv, nbb, (float*)m->grad.p,
+  hipLaunchKernelGGL(k_mlp_reduce, dim3(ceil_div(kNP, 16)), dim3(256), 0, ctx->stream,
+                     (const float*)m->part.p, nblk1, (const double*)lossv, nbb, (float*)m->grad.p,
                      d_loss);
   CHS_LAUNCH_CHECK(ctx);
   return CHS_OK;
