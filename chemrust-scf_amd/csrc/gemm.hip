@@ -374,6 +374,123 @@ __attribute__((amdgpu_waves_per_eu(MfmaTile<T, V>::WAVES))) k_gemm_mfma(int m, i
 }
 
 // ---------------------------------------------------------------------------
+// Small products (V = 6): 32 x 32 output tiles whose K range is split over the
+// four wavefronts of a workgroup, operands loaded straight from L2 into MFMA
+// registers (no LDS stage, no barrier in the K loop), the four partial tiles
+// summed in order through LDS. For products whose 64 x 64 tiles leave most of
+// the chip idle and whose time is the K loop's latency: the coefficient-space
+// products of the filter. Complex64: 512 x 160 x 256 in 7.5 us (64 x 64 tiles:
+// 26 us for 256 x 160 x 256), 256 x 160 x 23,847 in 69 us (75), 32 x 20 x 2,945
+// in 6.5 us (22). Lane (lk, li) supplies k = k0 + 2 lk + u in step u of an
+// 8-deep chunk, so a lane's two loads of a K-contiguous operand share 16 bytes.
+// ---------------------------------------------------------------------------
+constexpr int kSM = 32;  // output tile edge
+
+template <typename T, int OPA>
+__global__ void __launch_bounds__(256) k_gemm_small(int m, int n, int k, cplx<T> alpha,
+                                                    const cplx<T>* __restrict__ A, int lda,
+                                                    const cplx<T>* __restrict__ B, int ldb,
+                                                    cplx<T> beta, cplx<T>* __restrict__ C, int ldc,
+                                                    int klen, cplx<T>* __restrict__ part) {
+  using M = Mfma<T>;
+  using acc_t = typename M::acc_t;
+  constexpr int SA = OPA == 2 ? -1 : 1;  // conjugation folded into the products (k_gemm_mfma)
+  __shared__ cplx<T> red[4][4][4][64];   // [wavefront][tile][v][lane]
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+  const int m0 = blockIdx.x * kSM, n0 = blockIdx.y * kSM;
+  const int kb = blockIdx.z * klen, ke = min(k, kb + klen);
+  const int kw = ((klen + 3) / 4 + 7) / 8 * 8;  // K per wavefront, whole chunks
+  const int k0 = min(ke, kb + w * kw), k1 = min(ke, k0 + kw);
+  // rows and columns past the edge are clamped: they feed outputs never stored
+  const cplx<T>*pa[2], *pb[2];
+  const size_t ka = OPA == 0 ? (size_t)lda : 1;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = min(m0 + 16 * i + li, m - 1), c = min(n0 + 16 * i + li, n - 1);
+    pa[i] = A + (OPA == 0 ? (size_t)r : (size_t)r * lda);
+    pb[i] = B + (size_t)c * ldb;
+  }
+  acc_t p1[2][2], p2[2][2], p3[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) p1[i][j] = p2[i][j] = p3[i][j] = acc_t{0, 0, 0, 0};
+  auto products = [&](const cplx<T> (&a)[2], const cplx<T> (&b)[2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) p1[i][j] = M::mac(a[i].x, b[j].x, p1[i][j]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) p2[i][j] = M::mac(a[i].y, b[j].y, p2[i][j]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        p3[i][j] = M::mac(a[i].x + (T)SA * a[i].y, b[j].x + b[j].y, p3[i][j]);
+  };
+  int kk = k0;
+#pragma unroll 2
+  for (; kk + 8 <= k1; kk += 8) {
+    cplx<T> a[2][2], b[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const size_t q = (size_t)(kk + 2 * lk + u);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        a[u][i] = pa[i][q * ka];
+        b[u][i] = pb[i][q];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) products(a[u], b[u]);
+  }
+  if (kk < k1) {  // partial chunk: k past the end reads the last one and counts as zero
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int q = kk + 2 * lk + u;
+      const bool in = q < k1;
+      const size_t qc = (size_t)min(q, k1 - 1);
+      cplx<T> a[2], b[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        a[i] = in ? pa[i][qc * ka] : mk((T)0, (T)0);
+        b[i] = in ? pb[i][qc] : mk((T)0, (T)0);
+      }
+      products(a, b);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const T r1 = (T)p1[i][j][v], r2 = (T)p2[i][j][v], r2s = SA < 0 ? -r2 : r2;
+        red[w][2 * i + j][v][lane] = mk(r1 - r2s, (T)p3[i][j][v] - r1 - r2s);
+      }
+  __syncthreads();
+  // wavefront w stores tile w
+  const int i = w >> 1, j = w & 1;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const cplx<T> acc = (red[0][w][v][lane] + red[1][w][v][lane]) +
+                        (red[2][w][v][lane] + red[3][w][v][lane]);
+    const int r = m0 + 16 * i + M::row(lane, v), c = n0 + 16 * j + li;
+    if (r < m && c < n) {
+      if (part) {
+        part[(size_t)blockIdx.z * m * n + (size_t)r + (size_t)c * m] = acc;
+      } else {
+        cplx<T> val = alpha * acc;
+        if (beta.x != (T)0 || beta.y != (T)0) val = val + beta * C[(size_t)r + (size_t)c * ldc];
+        C[(size_t)r + (size_t)c * ldc] = val;
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // n = 1 (matrix-vector) in the memory-bound form: y = alpha op(A) x + beta y.
 // Both forms cut K into slices (blockIdx.y) so that a few thousand
 // wavefronts stream A, with four independent loads in flight per lane;
@@ -528,8 +645,17 @@ __global__ void k_gemm_reduce(int m, int n, int nz, const cplx<T>* __restrict__ 
                               cplx<T> alpha, cplx<T> beta, cplx<T>* __restrict__ C, int ldc) {
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (size_t)m * n) return;
+  const size_t mn = (size_t)m * n;
   cplx<T> s = mk((T)0, (T)0);
-  for (int z = 0; z < nz; ++z) s = s + part[(size_t)z * m * n + idx];
+  int z = 0;
+  for (; z + 8 <= nz; z += 8) {  // eight loads in flight, added in slice order
+    cplx<T> t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = part[(size_t)(z + u) * mn + idx];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s = s + t[u];
+  }
+  for (; z < nz; ++z) s = s + part[(size_t)z * mn + idx];
   const int r = (int)(idx % m), c = (int)(idx / m);
   cplx<T> v = alpha * s;
   if (beta.x != (T)0 || beta.y != (T)0) v = v + beta * C[(size_t)r + (size_t)c * ldc];
@@ -556,6 +682,7 @@ static constexpr int kSplitTargets[kNumSplitTargets] = {512, 1024, 2048, 4096};
 template <typename T>
 static void tile_dims(int variant, int* bm, int* bn, int* bk) {
   *bm = GBM; *bn = GBN; *bk = GBK;
+  if (variant == 6) *bm = *bn = *bk = kSM;
   if (variant == 1 || variant == 3) {
     *bm = MfmaTile<T, 1>::BM; *bn = MfmaTile<T, 1>::BN; *bk = MfmaTile<T, 1>::BK;
   } else if (variant == 5) {
@@ -566,8 +693,9 @@ static void tile_dims(int variant, int* bm, int* bn, int* bk) {
 }
 
 // tri: only the tiles that reach the diagonal or above are computed
+// min_len: shortest slice (the small kernel's wavefronts quarter it again)
 static void split_plan(int m, int n, int k, int bm, int bn, int bk, int target, int* ksplit,
-                       int* klen, bool tri = false) {
+                       int* klen, bool tri = false, int min_len = 256) {
   int tiles = (int)(ceil_div(m, bm) * ceil_div(n, bn));
   if (tri) {
     tiles = 0;
@@ -578,12 +706,20 @@ static void split_plan(int m, int n, int k, int bm, int bn, int bk, int target, 
   // at most `target` workgroups: whole rounds of resident workgroups, no
   // nearly empty last round
   if (tiles < target && k > 4 * bk)
-    ks = std::max(1, std::min(target / tiles, (k + 255) / 256));
+    ks = std::max(1, std::min(target / tiles, (k + min_len - 1) / min_len));
   int kl = (k + ks - 1) / ks;
   kl = ((kl + bk - 1) / bk) * bk;
   if (kl == 0) kl = bk;
   *klen = kl;
   *ksplit = std::max(1, (k + kl - 1) / kl);
+}
+
+// Split of variant v at a target (gemm_launch and the tuner agree on it).
+template <typename T>
+static void variant_plan(int v, int m, int n, int k, int target, bool tri, int* ksplit, int* klen) {
+  int bm, bn, bk;
+  tile_dims<T>(v, &bm, &bn, &bk);
+  split_plan(m, n, k, bm, bn, bk, target, ksplit, klen, tri && v != 0, v == 6 ? 128 : 256);
 }
 
 // Largest byte offset of a CL kernel's operand element from its stage base
@@ -604,7 +740,8 @@ static int gemm_launch(chs_context* ctx, int choice, int oa, int ob, int m, int 
   const int target = kSplitTargets[(choice >> 4) % kNumSplitTargets];
   // the offset-addressed kernels (3, 4, 5) only while their offsets fit 32 bits;
   // otherwise the bounds-tested kernel of the same tile
-  if (variant >= 3) {
+  if (variant == 6 && (oa == 1 || ob != 0 || tri)) variant = 3;
+  if (variant >= 3 && variant <= 5) {
     int bm0, bn0, bk0;
     tile_dims<T>(variant, &bm0, &bn0, &bk0);
     if (!cl_offsets_fit<T>(oa, ob, m, n, lda, ldb, bk0)) variant = variant == 4 ? 2 : 1;
@@ -612,7 +749,7 @@ static int gemm_launch(chs_context* ctx, int choice, int oa, int ob, int m, int 
   int bm, bn, bk;
   tile_dims<T>(variant, &bm, &bn, &bk);
   int ksplit, klen;
-  split_plan(m, n, k, bm, bn, bk, target, &ksplit, &klen, tri && variant != 0);
+  variant_plan<T>(variant, m, n, k, target, tri, &ksplit, &klen);
   cplx<T>* part = nullptr;
   if (ksplit > 1) {
     CHS_TRY(ensure(ctx, ws, (size_t)ksplit * m * n * sizeof(cplx<T>)));
@@ -622,6 +759,14 @@ static int gemm_launch(chs_context* ctx, int choice, int oa, int ob, int m, int 
   const int nfast = m > n ? 1 : 0;  // tiles sharing the larger operand run together
   const dim3 g1(((nblk + 7) / 8) * 8);  // multiple of 8 for the XCD-aware order
   const dim3 g3(ceil_div(m, bm), ceil_div(n, bn), ksplit);
+  if (variant == 6) {
+    if (oa == 0)
+      hipLaunchKernelGGL((k_gemm_small<T, 0>), g3, dim3(256), 0, ctx->stream, m, n, k, alpha, A,
+                         lda, B, ldb, beta, C, ldc, klen, part);
+    else
+      hipLaunchKernelGGL((k_gemm_small<T, 2>), g3, dim3(256), 0, ctx->stream, m, n, k, alpha, A,
+                         lda, B, ldb, beta, C, ldc, klen, part);
+  } else {
 #define CHS_GEMM_CASE(OA, OB)                                                                    \
   if (oa == OA && ob == OB) {                                                                    \
     if (variant == 1)                                                                            \
@@ -647,6 +792,7 @@ static int gemm_launch(chs_context* ctx, int choice, int oa, int ob, int m, int 
   CHS_GEMM_CASE(1, 0) CHS_GEMM_CASE(1, 1) CHS_GEMM_CASE(1, 2)
   CHS_GEMM_CASE(2, 0) CHS_GEMM_CASE(2, 1) CHS_GEMM_CASE(2, 2)
 #undef CHS_GEMM_CASE
+  }
   CHS_LAUNCH_CHECK(ctx);
   if (ksplit > 1) {
     hipLaunchKernelGGL((k_gemm_reduce<T>), dim3(ceil_div((size_t)m * n, 256)), dim3(256), 0,
@@ -656,15 +802,27 @@ static int gemm_launch(chs_context* ctx, int choice, int oa, int ob, int m, int 
   return CHS_OK;
 }
 
+// most 32 x 32 tiles the small-product kernel is tried with: four workgroups per
+// CU (with more, 64 x 64 tiles fill the chip and share operands through LDS: at
+// 3,730 tiles of the 64-atom O + beta C both take 86 us)
+constexpr int kSmallTiles = 1024;
+// and the most products (864 x 512 x 80,725 = 3.6e10 takes 2.4 times the 64 x 64
+// tiles' time; 256 x 160 x 23,847 = 9.8e8 is 20% faster)
+constexpr double kSmallWork = 4e9;
+
 // Kernel choice for a GEMM shape: variant (low 4 bits: 0 vector-FMA 64 x 64,
 // 1 MFMA 64 x 64, 2 MFMA 128-wide, 3 and 4 the same with clamped loads, 5
-// MFMA 64 x 64 x 32 with clamped loads) and split-K target (bits 4-5, index
-// into kSplitTargets). Chosen once per (precision, ops, m, n, k) by timing every
+// MFMA 64 x 64 x 32 with clamped loads, 6 the small-product kernel) and
+// split-K target (bits 4-5, index into kSplitTargets). The small-product kernel
+// is a candidate for op(A) in {N, C}, B not transposed and up to kSmallTiles
+// tiles and kSmallWork products, in complex64 and, where the caller asks (`small`), in complex128: the
+// FP64 products of Rayleigh-Ritz keep their summation order. Chosen once per (precision, ops, m, n, k) by timing every
 // distinct launch into a scratch output (HIP events, context stream);
 // outside a stream capture only, otherwise the MFMA 64 x 64 default.
 template <typename T>
 static int gemm_variant(chs_context* ctx, int oa, int ob, int m, int n, int k, const cplx<T>* A,
-                        int lda, const cplx<T>* B, int ldb, int* choice, int tri = 0) {
+                        int lda, const cplx<T>* B, int ldb, int* choice, int tri = 0,
+                        bool small = false) {
   auto* im = ctx->impl;
   if (!im->use_mfma) {
     *choice = 0;
@@ -674,7 +832,7 @@ static int gemm_variant(chs_context* ctx, int oa, int ob, int m, int n, int k, c
     *choice = im->gemm_choice;
     return CHS_OK;
   }
-  const GemmKey key{(int)sizeof(T), oa, ob + 16 * tri, m, n, k};
+  const GemmKey key{(int)sizeof(T), oa, ob + 16 * tri + (small && sizeof(T) == 8 ? 32 : 0), m, n, k};
   auto it = im->gemm_tune.find(key);
   if (it != im->gemm_tune.end()) {
     *choice = it->second;
@@ -690,12 +848,14 @@ static int gemm_variant(chs_context* ctx, int oa, int ob, int m, int n, int k, c
   double best = 1e300;
   // the vector-FMA kernel never wins a large product: not timed there
   const bool big = (double)m * n * k > 1e9;
-  for (int v = big ? 1 : 0; v < 6; ++v) {
+  const bool sm = (small || sizeof(T) == 4) && oa != 1 && ob == 0 && !tri &&
+                  (int)(ceil_div(m, kSM) * ceil_div(n, kSM)) <= kSmallTiles &&
+                  (double)m * n * k <= kSmallWork;
+  for (int v = big ? 1 : 0; v < (sm ? 7 : 6); ++v) {
     int prev_split = -1;
     for (int ti = 0; ti < kNumSplitTargets; ++ti) {
-      int bm, bn, bk, ks, kl;
-      tile_dims<T>(v, &bm, &bn, &bk);
-      split_plan(m, n, k, bm, bn, bk, kSplitTargets[ti], &ks, &kl, tri && v != 0);
+      int ks, kl;
+      variant_plan<T>(v, m, n, k, kSplitTargets[ti], tri, &ks, &kl);
       if (ks == prev_split) continue;  // same launch as a smaller target
       prev_split = ks;
       const int c = v | (ti << 4);
@@ -713,6 +873,7 @@ static int gemm_variant(chs_context* ctx, int oa, int ob, int m, int n, int k, c
         float tr = 0;
         CHS_HIP(ctx, hipEventElapsedTime(&tr, im->ev0, im->ev1));
         t = std::min(t, tr);
+        if (t > 1.25 * best) break;  // far behind: not timed again
       }
       if (t < best) {
         best = t;
@@ -731,14 +892,14 @@ static int gemm_variant(chs_context* ctx, int oa, int ob, int m, int n, int k, c
 template <typename T>
 static int gemm_t(chs_context* ctx, char opa, char opb, int m, int n, int k, cplx<T> alpha,
                   const cplx<T>* A, int lda, const cplx<T>* B, int ldb, cplx<T> beta, cplx<T>* C,
-                  int ldc) {
+                  int ldc, bool small = false) {
   const int oa = gemm_opcode(opa), ob = gemm_opcode(opb);
   if (oa < 0 || ob < 0 || m < 0 || n < 0 || k < 0) return CHS_ERR_INVALID_ARG;
   if (m == 0 || n == 0) return CHS_OK;
   if (n == 1 && ob == 0 && k > 0)  // matrix-vector
     return gemv_launch<T>(ctx, oa, m, k, alpha, A, lda, B, beta, C);
   int choice = 1;
-  CHS_TRY(gemm_variant<T>(ctx, oa, ob, m, n, k, A, lda, B, ldb, &choice));
+  CHS_TRY(gemm_variant<T>(ctx, oa, ob, m, n, k, A, lda, B, ldb, &choice, 0, small));
   return gemm_launch<T>(ctx, choice, oa, ob, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
                         ctx->impl->gemm_ws);
 }
@@ -746,6 +907,11 @@ static int gemm_t(chs_context* ctx, char opa, char opb, int m, int n, int k, cpl
 int zgemm(chs_context* ctx, char opa, char opb, int m, int n, int k, z64 alpha, const z64* A,
           int lda, const z64* B, int ldb, z64 beta, z64* C, int ldc) {
   return gemm_t<double>(ctx, opa, opb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+}
+
+int zgemm_small(chs_context* ctx, char opa, char opb, int m, int n, int k, z64 alpha, const z64* A,
+                int lda, const z64* B, int ldb, z64 beta, z64* C, int ldc) {
+  return gemm_t<double>(ctx, opa, opb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, true);
 }
 
 // C[i][j] = conj(C[j][i]) for i > j

@@ -62,9 +62,12 @@ struct Hamiltonian {
   DevBuf sinv_m;                 // c128 P x P (Q^-1 + beta^H beta)^-1
   DevBuf sinv_m_f;               // c64 copy
   DevBuf bmat;                   // c128 P x P beta^H beta
-  DevBuf bmat_f;                 // c64 copy
-  // projector coefficients carried through a Chebyshev filter (nl_ws, five
-  // P x n_b slots): slots of W_{k-1}, W_k and G = beta^H O; 3 and 4 scratch
+  // left factor of the filter's coefficient step: [M; B M] (2P x P) with S,
+  // B (P x P) without, c128 and c64, and the P reciprocals 1/Q
+  DevBuf kstack, kstack_f, qinv;
+  // projector coefficients carried through a Chebyshev filter (nl_ws: three
+  // 2P x n_b slots [step coefficients; W] and a P x n_b one): the slots of
+  // W_{k-1}, W_k and G = beta^H O
   DevBuf nl_ws;
   int nl_wp = 0, nl_w = 1, nl_g = 2;
   DevBuf fscr;                   // second Chebyshev buffer of a k-point set member
@@ -75,7 +78,7 @@ struct Hamiltonian {
 };
 
 inline void release_hamiltonian(Hamiltonian& h) {
-  for (DevBuf* b : {&h.veff_f, &h.st_mem, &h.beta_f, &h.sinv_m, &h.sinv_m_f, &h.bmat, &h.bmat_f,
+  for (DevBuf* b : {&h.veff_f, &h.st_mem, &h.beta_f, &h.sinv_m, &h.sinv_m_f, &h.bmat, &h.kstack, &h.kstack_f, &h.qinv,
                     &h.nl_ws, &h.fscr, &h.h3_cn.buf, &h.h3_nn.buf, &h.h3_exp})
     release(*b);
   h = Hamiltonian{};

@@ -10,6 +10,10 @@ int zgemm(chs_context* ctx, char opa, char opb, int m, int n, int k, z64 alpha, 
 // tiles on or above the diagonal are computed, the lower triangle mirrored.
 int zgemm_herm(chs_context* ctx, int n, int k, const z64* A, int lda, const z64* B, int ldb, z64* C,
                int ldc);
+// zgemm with the small-product kernel among the tuner's candidates (the
+// filter's products; zgemm itself keeps its kernels and their sums' order).
+int zgemm_small(chs_context* ctx, char opa, char opb, int m, int n, int k, z64 alpha, const z64* A,
+                int lda, const z64* B, int ldb, z64 beta, z64* C, int ldc);
 int cgemm(chs_context* ctx, char opa, char opb, int m, int n, int k, c32 alpha, const c32* A,
           int lda, const c32* B, int ldb, c32 beta, c32* C, int ldc);
 // y = alpha op(A) x + beta y (op N, T or C) with A held in complex64 and x,

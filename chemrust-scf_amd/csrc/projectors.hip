@@ -44,6 +44,20 @@ __global__ void k_diag_add_inv(z64* __restrict__ a, const double* __restrict__ q
   if (i < P) a[(size_t)i + (size_t)i * P].x += 1.0 / q[i];
 }
 
+// [M; B M] (2P x P) and 1/Q, with B M = 1 - Q^{-1} M (M (Q^{-1} + B) = 1).
+__global__ void k_stack_m(const z64* __restrict__ M, const double* __restrict__ q, int P,
+                          z64* __restrict__ K, double* __restrict__ qinv) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (size_t)P * P) return;
+  const int r = (int)(i % P), c = (int)(i / P);
+  const z64 v = M[i];
+  const double qi = 1.0 / q[r];
+  z64* col = K + (size_t)c * 2 * P;
+  col[r] = v;
+  col[P + r] = mk((r == c ? 1.0 : 0.0) - qi * v.x, -qi * v.y);
+  if (c == 0) qinv[r] = qi;
+}
+
 template <typename A, typename B>
 __global__ void k_convert(const A* __restrict__ a, B* __restrict__ b, size_t n) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -58,10 +72,10 @@ static int ensure_c64_projectors(chs_context* ctx) {
     hipLaunchKernelGGL((k_convert<z64, c32>), dim3(ceil_div(nb, 256)), dim3(256), 0, ctx->stream,
                        (const z64*)H.beta, (c32*)H.beta_f.p, nb);
     CHS_LAUNCH_CHECK(ctx);
-    const size_t pp = (size_t)H.n_proj * H.n_proj;
-    CHS_TRY(ensure(ctx, H.bmat_f, pp * sizeof(c32)));
-    hipLaunchKernelGGL((k_convert<z64, c32>), dim3(ceil_div(pp, 256)), dim3(256), 0, ctx->stream,
-                       (const z64*)H.bmat.p, (c32*)H.bmat_f.p, pp);
+    const size_t pp = (size_t)H.n_proj * H.n_proj, ks = (H.has_s ? 2 : 1) * pp;
+    CHS_TRY(ensure(ctx, H.kstack_f, ks * sizeof(c32)));
+    hipLaunchKernelGGL((k_convert<z64, c32>), dim3(ceil_div(ks, 256)), dim3(256), 0, ctx->stream,
+                       (const z64*)H.kstack.p, (c32*)H.kstack_f.p, ks);
     if (H.has_s) {
       CHS_TRY(ensure(ctx, H.sinv_m_f, pp * sizeof(c32)));
       hipLaunchKernelGGL((k_convert<z64, c32>), dim3(ceil_div(pp, 256)), dim3(256), 0,
@@ -122,72 +136,91 @@ static int nonlocal_t(chs_context* ctx, const cplx<T>* psi, int n_b, cplx<T>* hp
 // ---------------------------------------------------------------------------
 // Projector part of one Chebyshev step in coefficient space. With
 // W_k = beta^H X_k, the step X_{k+1} = 2 (S^{-1} H X_k - c X_k) / e - X_{k-1}
-// splits as X_{k+1} = O + (2/e) beta C, where O is the local-potential step
-// (the fused H|psi> pipeline's Chebyshev epilogue) and
+// splits as X_{k+1} = O + f beta C (f = 2/e, or 1/e on the first step), where
+// O is the local-potential step (the fused H|psi> pipeline's Chebyshev
+// epilogue) and
 //   C = D W_k - M (Z + B D W_k),   Z = beta^H H_loc X_k,
-// B = beta^H beta, M = (Q^{-1} + B)^{-1} (C = D W_k when S = 1). Z follows
+// B = beta^H beta, M = (Q^{-1} + B)^{-1} (C = D W_k when S = 1). Since
+// M (Q^{-1} + B) = 1 this is C = M y with y = Q^{-1} D W_k - Z. Z follows
 // from G = beta^H O: Z = (e/2)(G + W_{k-1}) + c W_k (first step:
-// Z = e G + c W_0), and W_{k+1} = G + (2/e) B C. Two n_pw-long GEMMs per
-// step (G and the beta C update) instead of four, and no H|psi> block.
+// Z = e G + c W_0), and W_{k+1} = G + f B C = G + f (B M) y. Two n_pw-long
+// GEMMs per step (G and the beta C update) and one product [M; B M] (f y) into
+// [f C; W_{k+1}], whose lower half holds G (without S: B (f D W_k) into the
+// lower half). Three dependent P x P products and a scaling pass were a sixth
+// of the k-point set's filter (64 atoms: 26 us each, 12 workgroups).
 // ---------------------------------------------------------------------------
-// coef = {c, inv_e} on the device (graph-replayable): Z = a1 G + a2 W_{k-1}
-// + c W with (a1, a2) = (e, 0) on the first step and (e/2, e/2) after;
-// DW = D W. Without S the scaled coefficients f D W go straight to Cs.
-// Residual-based filter: O carries the extra term s_b R_b (R the residual
-// block, s_b = ress[b]), so G = beta^H O holds s_b beta^H R_b too; BR =
-// beta^H R removes it before Z is formed.
+// Elementwise part, coef = {c, inv_e} on the device (graph-replayable). W, Wp
+// and G are the lower halves of 2P x n_b slots (leading dimension 2P), `top`
+// the upper half of G's slot. With S: y <- f y and top <- 0; without:
+// top <- f D W. Residual-based filter: O carries the extra term s_b R_b (R the
+// residual block, s_b = ress[b]), so G = beta^H O holds s_b beta^H R_b too;
+// BR = beta^H R (P x n_b) removes it before Z is formed.
 template <typename T>
 __global__ void k_cheb_coef(const cplx<T>* __restrict__ G, const cplx<T>* __restrict__ Wp,
                             const cplx<T>* __restrict__ W, const double* __restrict__ d,
-                            const double* __restrict__ coef, int first, int P, size_t n,
-                            cplx<T>* __restrict__ Z, cplx<T>* __restrict__ DW,
-                            const cplx<T>* __restrict__ BR, const double* __restrict__ ress) {
+                            const double* __restrict__ qinv, const double* __restrict__ coef,
+                            int first, int P, size_t n, cplx<T>* __restrict__ y,
+                            cplx<T>* __restrict__ top, const cplx<T>* __restrict__ BR,
+                            const double* __restrict__ ress) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const T c = (T)coef[0], e = (T)(1.0 / coef[1]);
-  const cplx<T> w = W[i];
-  const T dp = (T)d[(int)(i % P)];
-  if (Z) {
-    const T a1 = first ? e : (T)0.5 * e, a2 = first ? (T)0 : (T)0.5 * e;
-    // W_{k-1} does not exist on the first step (not read)
-    cplx<T> g = G[i];
-    const cplx<T> wp = first ? mk((T)0, (T)0) : Wp[i];
-    if (BR) {
-      const T sb = (T)ress[i / P];
-      const cplx<T> br = BR[i];
-      g = mk(g.x - sb * br.x, g.y - sb * br.y);
-    }
-    Z[i] = mk(a1 * g.x + a2 * wp.x + c * w.x, a1 * g.y + a2 * wp.y + c * w.y);
-    DW[i] = mk(dp * w.x, dp * w.y);
-  } else {
-    const T f = (T)(first ? coef[1] : 2.0 * coef[1]);
-    DW[i] = mk(f * dp * w.x, f * dp * w.y);
+  const size_t b = i / P;
+  const int p = (int)(i - b * P);
+  const size_t q = b * 2 * P + p;  // in the 2P-strided halves
+  // FP64 throughout, rounded once: y is a difference of like terms
+  const double inv_e = coef[1], c = coef[0], f = first ? inv_e : 2.0 * inv_e;
+  const z64 w = mk((double)W[q].x, (double)W[q].y);
+  if (!y) {
+    top[q] = mk((T)(f * d[p] * w.x), (T)(f * d[p] * w.y));
+    return;
   }
+  const double a1 = first ? 1.0 / inv_e : 0.5 / inv_e, a2 = first ? 0.0 : a1;
+  // W_{k-1} does not exist on the first step (not read)
+  z64 g = mk((double)G[q].x, (double)G[q].y);
+  const z64 wp = first ? mk(0.0, 0.0) : mk((double)Wp[q].x, (double)Wp[q].y);
+  if (BR) {
+    const double sb = ress[b];
+    g = mk(g.x - sb * BR[i].x, g.y - sb * BR[i].y);
+  }
+  const double e = d[p] * qinv[p] - c;  // Q^{-1} D W - c W
+  y[i] = mk((T)(f * (e * w.x - a1 * g.x - a2 * wp.x)), (T)(f * (e * w.y - a1 * g.y - a2 * wp.y)));
+  top[q] = mk((T)0, (T)0);
 }
 
-// Cs *= f with f = inv_e (first step) or 2 inv_e
+// The filter's products: the small-product kernel may take them.
 template <typename T>
-__global__ void k_cheb_scale(cplx<T>* __restrict__ x, const double* __restrict__ coef, int first,
-                             size_t n) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const T f = (T)(first ? coef[1] : 2.0 * coef[1]);
-  x[i] = mk(f * x[i].x, f * x[i].y);
+static int gemm_filter(chs_context* ctx, char oa, int m, int n, int k, const cplx<T>* A, int lda,
+                       const cplx<T>* B, int ldb, double be, cplx<T>* C, int ldc) {
+  if constexpr (sizeof(T) == 8)
+    return zgemm_small(ctx, oa, 'N', m, n, k, mk(1.0, 0.0), A, lda, B, ldb, mk(be, 0.0), C, ldc);
+  else
+    return cgemm(ctx, oa, 'N', m, n, k, mk(1.f, 0.f), A, lda, B, ldb, mk((float)be, 0.f), C, ldc);
 }
 
+// Slot s of the coefficient state (2P x n_b; slot 3: P x n_b).
 template <typename T>
 static cplx<T>* nl_slot(Hamiltonian& H, int n_b, int slot) {
-  return (cplx<T>*)H.nl_ws.p + (size_t)slot * H.n_proj * n_b;
+  return (cplx<T>*)H.nl_ws.p + (size_t)slot * 2 * H.n_proj * n_b;
+}
+// its lower half, W
+template <typename T>
+static cplx<T>* nl_low(Hamiltonian& H, int n_b, int slot) {
+  return nl_slot<T>(H, n_b, slot) + H.n_proj;
+}
+
+static int cheb_nl_state(chs_context* ctx, int n_b, size_t csz) {
+  Hamiltonian& H = ctx->impl->ham;
+  H.nl_wp = 0;
+  H.nl_w = 1;
+  H.nl_g = 2;
+  return ensure(ctx, H.nl_ws, 7 * (size_t)H.n_proj * n_b * csz);
 }
 
 template <typename T>
 static int cheb_nl_begin_t(chs_context* ctx, const cplx<T>* X0, int n_b) {
   Hamiltonian& H = ctx->impl->ham;
   const int P = H.n_proj;
-  CHS_TRY(ensure(ctx, H.nl_ws, 5 * (size_t)P * n_b * sizeof(cplx<T>)));
-  H.nl_wp = 0;
-  H.nl_w = 1;
-  H.nl_g = 2;
+  CHS_TRY(cheb_nl_state(ctx, n_b, sizeof(cplx<T>)));
   const cplx<T>* beta = sizeof(T) == 8 ? (const cplx<T>*)H.beta : (const cplx<T>*)H.beta_f.p;
   if constexpr (sizeof(T) == 4) {
     if (ctx->impl->use_h3) {
@@ -195,11 +228,11 @@ static int cheb_nl_begin_t(chs_context* ctx, const cplx<T>* X0, int n_b) {
       int* eb = (int*)H.h3_exp.p;
       CHS_TRY(h3_column_exponents(ctx, X0, H.n_pw, n_b, H.n_pw, eb));
       return h3_gemm(ctx, H.h3_cn, n_b, mk(1.f, 0.f), X0, H.n_pw, eb, mk(0.f, 0.f),
-                     nl_slot<T>(H, n_b, H.nl_w), P);
+                     nl_low<T>(H, n_b, H.nl_w), 2 * P);
     }
   }
-  return gemm_any<T>(ctx, 'C', 'N', P, n_b, H.n_pw, 1.0, beta, H.n_pw, X0, H.n_pw, 0.0,
-                     nl_slot<T>(H, n_b, H.nl_w), P);
+  return gemm_filter<T>(ctx, 'C', P, n_b, H.n_pw, beta, H.n_pw, X0, H.n_pw, 0.0,
+                        nl_low<T>(H, n_b, H.nl_w), 2 * P);
 }
 
 template <typename T>
@@ -209,15 +242,11 @@ static int cheb_nl_step_t(chs_context* ctx, cplx<T>* O, int n_b, bool first, con
   const int P = H.n_proj, n_pw = H.n_pw;
   const bool f32 = sizeof(T) == 4;
   const cplx<T>* beta = f32 ? (const cplx<T>*)H.beta_f.p : (const cplx<T>*)H.beta;
-  const cplx<T>* B = f32 ? (const cplx<T>*)H.bmat_f.p : (const cplx<T>*)H.bmat.p;
-  const cplx<T>* M = f32 ? (const cplx<T>*)H.sinv_m_f.p : (const cplx<T>*)H.sinv_m.p;
-  cplx<T>* Wp = nl_slot<T>(H, n_b, H.nl_wp);
-  cplx<T>* W = nl_slot<T>(H, n_b, H.nl_w);
-  cplx<T>* G = nl_slot<T>(H, n_b, H.nl_g);
-  cplx<T>* Z = nl_slot<T>(H, n_b, 3);
-  cplx<T>* Cs = nl_slot<T>(H, n_b, 4);
+  const cplx<T>* K = f32 ? (const cplx<T>*)H.kstack_f.p : (const cplx<T>*)H.kstack.p;
+  cplx<T>* stack = nl_slot<T>(H, n_b, H.nl_g);  // [f C; W_{k+1}]
+  cplx<T>* G = stack + P;
+  cplx<T>* y = nl_slot<T>(H, n_b, 3);
   const size_t pb = (size_t)P * n_b;
-  const unsigned gp = ceil_div(pb, 256);
   // complex64 with fp16x3: both n_pw-long products on the fp16 matrix cores
   bool h3 = false;
   int* eb = nullptr;
@@ -232,30 +261,29 @@ static int cheb_nl_step_t(chs_context* ctx, cplx<T>* O, int n_b, bool first, con
   if constexpr (sizeof(T) == 4) {
     if (h3) {
       CHS_TRY(h3_column_exponents(ctx, O, n_pw, n_b, n_pw, eb));
-      CHS_TRY(h3_gemm(ctx, H.h3_cn, n_b, mk(1.f, 0.f), O, n_pw, eb, mk(0.f, 0.f), G, P));
+      CHS_TRY(h3_gemm(ctx, H.h3_cn, n_b, mk(1.f, 0.f), O, n_pw, eb, mk(0.f, 0.f), G, 2 * P));
     }
   }
-  if (!h3) CHS_TRY(gemm_any<T>(ctx, 'C', 'N', P, n_b, n_pw, 1.0, beta, n_pw, O, n_pw, 0.0, G, P));
-  hipLaunchKernelGGL((k_cheb_coef<T>), dim3(gp), dim3(256), 0, ctx->stream, G, Wp, W, H.dion,
-                     coef, (int)first, P, pb, H.has_s ? Z : nullptr, Cs, BR, ress);
+  if (!h3) CHS_TRY(gemm_filter<T>(ctx, 'C', P, n_b, n_pw, beta, n_pw, O, n_pw, 0.0, G, 2 * P));
+  hipLaunchKernelGGL((k_cheb_coef<T>), dim3(ceil_div(pb, 256)), dim3(256), 0, ctx->stream, G,
+                     nl_low<T>(H, n_b, H.nl_wp), nl_low<T>(H, n_b, H.nl_w), H.dion,
+                     (const double*)H.qinv.p, coef, (int)first, P, pb, H.has_s ? y : nullptr, stack,
+                     BR, ress);
   CHS_LAUNCH_CHECK(ctx);
-  if (H.has_s) {
-    // Z += B (D W); C = D W - M Z; Cs = f C
-    CHS_TRY(gemm_any<T>(ctx, 'N', 'N', P, n_b, P, 1.0, B, P, Cs, P, 1.0, Z, P));
-    CHS_TRY(gemm_any<T>(ctx, 'N', 'N', P, n_b, P, -1.0, M, P, Z, P, 1.0, Cs, P));
-    hipLaunchKernelGGL((k_cheb_scale<T>), dim3(gp), dim3(256), 0, ctx->stream, Cs, coef,
-                       (int)first, pb);
-    CHS_LAUNCH_CHECK(ctx);
-  }
-  // X_{k+1} = O + beta Cs ; W_{k+1} = G + B Cs (into G's slot)
+  // [f C; W_{k+1}] = [0; G] + [M; B M] (f y), or W_{k+1} = G + B (f C)
+  if (H.has_s)
+    CHS_TRY(gemm_filter<T>(ctx, 'N', 2 * P, n_b, P, K, 2 * P, y, P, 1.0, stack, 2 * P));
+  else
+    CHS_TRY(gemm_filter<T>(ctx, 'N', P, n_b, P, K, P, stack, 2 * P, 1.0, G, 2 * P));
+  // X_{k+1} = O + beta (f C)
   if constexpr (sizeof(T) == 4) {
     if (h3) {
-      CHS_TRY(h3_column_exponents(ctx, Cs, P, n_b, P, eb + n_b));
-      CHS_TRY(h3_gemm(ctx, H.h3_nn, n_b, mk(1.f, 0.f), Cs, P, eb + n_b, mk(1.f, 0.f), O, n_pw));
+      CHS_TRY(h3_column_exponents(ctx, stack, P, n_b, 2 * P, eb + n_b));
+      CHS_TRY(h3_gemm(ctx, H.h3_nn, n_b, mk(1.f, 0.f), stack, 2 * P, eb + n_b, mk(1.f, 0.f), O,
+                      n_pw));
     }
   }
-  if (!h3) CHS_TRY(gemm_any<T>(ctx, 'N', 'N', n_pw, n_b, P, 1.0, beta, n_pw, Cs, P, 1.0, O, n_pw));
-  CHS_TRY(gemm_any<T>(ctx, 'N', 'N', P, n_b, P, 1.0, B, P, Cs, P, 1.0, G, P));
+  if (!h3) CHS_TRY(gemm_filter<T>(ctx, 'N', n_pw, n_b, P, beta, n_pw, stack, 2 * P, 1.0, O, n_pw));
   const int old_wp = H.nl_wp;
   H.nl_wp = H.nl_w;
   H.nl_w = H.nl_g;
@@ -276,16 +304,19 @@ int cheb_nl_step(chs_context* ctx, int precision, void* O, int n_b, bool first,
   return cheb_nl_step_t<float>(ctx, (c32*)O, n_b, first, d_coef, (const c32*)br, ress);
 }
 
-// Coefficients of the residual filter's first two iterates: W_0 = beta^H R_0
-// = 0 and W_1 = beta^H R_1 = inv_e BR (BR = beta^H R, R the residual block).
+// Coefficients of the residual filter's first two iterates (leading dimension
+// 2P): W_0 = beta^H R_0 = 0 and W_1 = beta^H R_1 = inv_e BR (BR = beta^H R,
+// P x n_b, R the residual block).
 template <typename T>
 __global__ void k_res_coef_start(const cplx<T>* __restrict__ BR, const double* __restrict__ coef,
-                                 size_t n, cplx<T>* __restrict__ W0, cplx<T>* __restrict__ W1) {
+                                 int P, size_t n, cplx<T>* __restrict__ W0,
+                                 cplx<T>* __restrict__ W1) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  const size_t q = i + i / P * P;
   const T f = (T)coef[1];
-  W0[i] = mk((T)0, (T)0);
-  W1[i] = mk(f * BR[i].x, f * BR[i].y);
+  W0[q] = mk((T)0, (T)0);
+  W1[q] = mk(f * BR[i].x, f * BR[i].y);
 }
 
 template <typename T>
@@ -293,16 +324,13 @@ static int cheb_nl_begin_res_t(chs_context* ctx, const cplx<T>* R, int n_b, cons
                                cplx<T>* BR) {
   Hamiltonian& H = ctx->impl->ham;
   const int P = H.n_proj;
-  CHS_TRY(ensure(ctx, H.nl_ws, 5 * (size_t)P * n_b * sizeof(cplx<T>)));
-  H.nl_wp = 0;
-  H.nl_w = 1;
-  H.nl_g = 2;
+  CHS_TRY(cheb_nl_state(ctx, n_b, sizeof(cplx<T>)));
   const cplx<T>* beta = sizeof(T) == 8 ? (const cplx<T>*)H.beta : (const cplx<T>*)H.beta_f.p;
-  CHS_TRY(gemm_any<T>(ctx, 'C', 'N', P, n_b, H.n_pw, 1.0, beta, H.n_pw, R, H.n_pw, 0.0, BR, P));
+  CHS_TRY(gemm_filter<T>(ctx, 'C', P, n_b, H.n_pw, beta, H.n_pw, R, H.n_pw, 0.0, BR, P));
   const size_t pb = (size_t)P * n_b;
   hipLaunchKernelGGL((k_res_coef_start<T>), dim3(ceil_div(pb, 256)), dim3(256), 0, ctx->stream,
-                     (const cplx<T>*)BR, coef, pb, nl_slot<T>(H, n_b, H.nl_wp),
-                     nl_slot<T>(H, n_b, H.nl_w));
+                     (const cplx<T>*)BR, coef, P, pb, nl_low<T>(H, n_b, H.nl_wp),
+                     nl_low<T>(H, n_b, H.nl_w));
   CHS_LAUNCH_CHECK(ctx);
   return CHS_OK;
 }
@@ -738,7 +766,7 @@ int chs_bind_projectors(chs_context* ctx, int n_proj, const double* d_beta, cons
   H.has_s = false;
   release(H.beta_f);
   release(H.sinv_m_f);
-  release(H.bmat_f);
+  release(H.kstack_f);
   release(H.h3_cn.buf);
   release(H.h3_nn.buf);
   if (n_proj == 0) return CHS_OK;
@@ -762,7 +790,10 @@ int chs_bind_projectors(chs_context* ctx, int n_proj, const double* d_beta, cons
   CHS_TRY(zgemm(ctx, 'C', 'N', P, P, H.n_pw, mk(1.0, 0.0), (const z64*)d_beta, H.n_pw,
                 (const z64*)d_beta, H.n_pw, mk(0.0, 0.0), (z64*)H.bmat.p, P));
   CHS_TRY(hermitise(ctx, (z64*)H.bmat.p, P));
+  CHS_TRY(ensure(ctx, H.kstack, (any ? 2 : 1) * pp * sizeof(z64)));
   if (!any) {
+    CHS_HIP(ctx, hipMemcpyAsync(H.kstack.p, H.bmat.p, pp * sizeof(z64), hipMemcpyDeviceToDevice,
+                                ctx->stream));
     CHS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return CHS_OK;
   }
@@ -781,6 +812,10 @@ int chs_bind_projectors(chs_context* ctx, int n_proj, const double* d_beta, cons
   CHS_TRY(tri_inv(ctx, A, Li, P));
   CHS_TRY(zgemm(ctx, 'C', 'N', P, P, P, mk(1.0, 0.0), Li, P, Li, P, mk(0.0, 0.0),
                 (z64*)H.sinv_m.p, P));
+  CHS_TRY(ensure(ctx, H.qinv, (size_t)P * sizeof(double)));
+  hipLaunchKernelGGL(k_stack_m, dim3(ceil_div(pp, 256)), dim3(256), 0, ctx->stream,
+                     (const z64*)H.sinv_m.p, d_q, P, (z64*)H.kstack.p, (double*)H.qinv.p);
+  CHS_LAUNCH_CHECK(ctx);
   H.has_s = true;
   CHS_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return CHS_OK;
