@@ -614,7 +614,7 @@ static int gemv_launch(chs_context* ctx, int oa, int m, int k, cplx<T> alpha, co
                        int lda, const cplx<T>* x, cplx<T> beta, cplx<T>* y) {
   int ns, klen;
   if (oa == 0)
-    gemv_plan(k, (int)ceil_div(m, 64), 16, &ns, &klen);
+    gemv_plan(k, (int)ceil_div(m, 64), 64, &ns, &klen);  // short rows: no second launch
   else
     gemv_plan(k, m, 512, &ns, &klen);
   cplx<T>* part = nullptr;

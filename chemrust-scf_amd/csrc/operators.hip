@@ -1,5 +1,6 @@
 // Operator entry points: H|psi>, the Chebyshev filter, spectral bounds and
 // the Lanczos upper bound; level-1 primitives.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -32,25 +33,69 @@ int apply_h_impl(chs_context* ctx, int precision, const void* psi, int n_b, void
   return CHS_OK;
 }
 
-__global__ void k_norm_guard2(const double* __restrict__ part, int n_part, int k,
-                              double* __restrict__ flag) {
-  __shared__ double sh[8];
-  double a = 0, b = 0;
-  for (int i = threadIdx.x; i < n_part; i += blockDim.x) {
-    a += part[2 * i];
-    b += part[2 * i + 1];
-  }
-  double r = block_sum(a, sh);
-  double s = block_sum(b, sh);
+// Threads of the one-block reductions (the norm guards and the Lanczos vector
+// kernels): 16 wavefronts, so that a lone workgroup keeps enough loads in flight
+// (10,080 guard partials: 13.6 us with 256 threads, 5.3 us with 1024).
+constexpr int kOneBlock = 1024;
+
+// Sum over a workgroup of up to 16 wavefronts, visible to every thread
+// (sh: 17 doubles).
+__device__ __forceinline__ double one_block_sum(double v, double* sh) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
   if (threadIdx.x == 0) {
-    const double nc = sqrt(r), np = sqrt(s);
-    const double growth = np > 0.0 ? nc / np : 1.0;
-    if (flag[0] == 0.0 && growth > 10.0) {
-      flag[0] = k;
-      flag[1] = np;
-      flag[2] = nc;
-      flag[3] = growth;
-    }
+    double r = 0;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) r += sh[w];
+    sh[16] = r;
+  }
+  __syncthreads();
+  const double r = sh[16];
+  __syncthreads();
+  return r;
+}
+
+// The growth guard: previous norm^2 s, current r; the first step whose growth
+// exceeds 10 is kept in flag[0..3].
+__device__ __forceinline__ void guard_check(double r, double s, int k, double* __restrict__ flag) {
+  const double nc = sqrt(r), np = sqrt(s);
+  const double growth = np > 0.0 ? nc / np : 1.0;
+  if (flag[0] == 0.0 && growth > 10.0) {
+    flag[0] = k;
+    flag[1] = np;
+    flag[2] = nc;
+    flag[3] = growth;
+  }
+}
+
+__global__ void __launch_bounds__(kOneBlock) k_norm_guard2(const double2* __restrict__ part,
+                                                           int n_part, int k,
+                                                           double* __restrict__ flag) {
+  __shared__ double sh[17];
+  double a = 0, b = 0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n_part; i += kOneBlock) {
+    const double2 p = part[i];
+    a += p.x;
+    b += p.y;
+  }
+  const double r = one_block_sum(a, sh), s = one_block_sum(b, sh);
+  if (threadIdx.x == 0) guard_check(r, s, k, flag);
+}
+
+// The rolling guard on the previous iterate, whose |p|^2 partials the forward z
+// pass of this step leaves (flag[4] keeps the last norm^2).
+__global__ void __launch_bounds__(kOneBlock) k_norm_guard_prev(const double2* __restrict__ part,
+                                                               int n_part, int k, int first,
+                                                               double* __restrict__ flag) {
+  __shared__ double sh[17];
+  double a = 0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n_part; i += kOneBlock) a += part[i].y;
+  const double r = one_block_sum(a, sh);
+  if (threadIdx.x == 0) {
+    if (!first) guard_check(r, flag[4], k, flag);
+    flag[4] = r;
   }
 }
 
@@ -69,8 +114,7 @@ __global__ void __launch_bounds__(kRedThreads) k_sqnorm_part(const cplx<T>* __re
 }
 
 // Growth guard on consecutive iterates: flag[4] keeps |Y_{k-1}|^2 of the
-// previous step; from the second step on, growth > 10 sets flag[0..3] as
-// k_norm_guard2 does.
+// previous step; from the second step on the guard compares with it.
 __global__ void k_norm_guard_roll(const double* __restrict__ part, int n_part, int k, int first,
                                   double* __restrict__ flag) {
   __shared__ double sh[8];
@@ -78,64 +122,81 @@ __global__ void k_norm_guard_roll(const double* __restrict__ part, int n_part, i
   for (int i = threadIdx.x; i < n_part; i += blockDim.x) a += part[i];
   const double r = block_sum(a, sh);
   if (threadIdx.x == 0) {
-    if (!first) {
-      const double nc = sqrt(r), np = sqrt(flag[4]);
-      const double growth = np > 0.0 ? nc / np : 1.0;
-      if (flag[0] == 0.0 && growth > 10.0) {
-        flag[0] = k;
-        flag[1] = np;
-        flag[2] = nc;
-        flag[3] = growth;
-      }
-    }
+    if (!first) guard_check(r, flag[4], k, flag);
     flag[4] = r;
   }
+}
+
+constexpr int kNormBlocks = 2048;
+
+// Norm partials of a filter: {|out|^2, |in|^2} per block of the forward z pass
+// (at its smallest stick chunk) or one per workgroup of the last norm.
+static size_t cheb_part_bytes(chs_context* ctx, int n_b) {
+  const size_t gz = ceil_div(ctx->impl->ham.st.n_st, 16);
+  return sizeof(double) * std::max<size_t>(2 * gz * n_b, kNormBlocks) + 64;
 }
 
 // One Chebyshev step Y_out = [2] (A Y_in - c Y_in)/e [- Y_prev] with the
 // growth guard; A = H (fused epilogue) or S^{-1} H (projector path). With a
 // residual block (resw, per-band scales ress, its projector coefficients br)
-// the step is the residual filter's, Y_out += ress[b] resw_b; guard_first
-// then marks the first step the growth guard sees.
+// the step is the residual filter's, Y_out += ress[b] resw_b. With projectors
+// the guard runs one step behind, on the norms of yin that the forward z pass
+// sums anyway, and cheb_guard_last takes the last iterate: no pass over the
+// block for its norm alone (216 atoms: 58 us a step).
 static int cheb_step(chs_context* ctx, int precision, const void* yin, int n_b, void* yout,
                      const void* yprev, bool first, const double* d_coef, int k, double* flag,
                      const void* resw = nullptr, const double* ress = nullptr,
-                     const void* br = nullptr, bool guard_first = false) {
+                     const void* br = nullptr) {
   Hamiltonian& H = ctx->impl->ham;
   auto* im = ctx->impl;
-  const size_t ne = (size_t)n_b * H.n_pw;
   const int mode = resw ? EPI_CHEBK_RES : first ? EPI_CHEB1 : EPI_CHEBK;
   if (resw) first = false;
   if (H.n_proj == 0) {
-    const int gz = ceil_div(H.st.n_st, 16);  // partials of the smallest stick chunk
-    CHS_TRY(ensure(ctx, im->part, sizeof(double) * 2 * (size_t)gz * n_b + 64));
+    CHS_TRY(ensure(ctx, im->part, cheb_part_bytes(ctx, n_b)));
     int n_part = 0;
     CHS_TRY(vloc_pipeline(ctx, precision, yin, n_b, yout, mode, yprev, d_coef, 0.0, 0.0,
                           (double*)im->part.p, &n_part, resw, ress));
     if (!first) {
-      hipLaunchKernelGGL(k_norm_guard2, dim3(1), dim3(256), 0, ctx->stream,
-                         (const double*)im->part.p, n_part, k, flag);
+      hipLaunchKernelGGL(k_norm_guard2, dim3(1), dim3(kOneBlock), 0, ctx->stream,
+                         (const double2*)im->part.p, n_part, k, flag);
       CHS_LAUNCH_CHECK(ctx);
     }
     return CHS_OK;
   }
-  // projector path: the local step with the fused epilogue, then the
-  // projector terms in coefficient space (cheb_nl_step), then the norm
-  CHS_TRY(vloc_pipeline(ctx, precision, yin, n_b, yout, mode, yprev, d_coef, 0.0, 0.0, nullptr,
-                        nullptr, resw, ress));
-  CHS_TRY(cheb_nl_step(ctx, precision, yout, n_b, first, d_coef, resw ? br : nullptr, ress));
-  // |Y_k|^2 over the whole block: enough workgroups to stream it at HBM rate
-  constexpr int kNormBlocks = 2048;
-  CHS_TRY(ensure(ctx, im->part, sizeof(double) * kNormBlocks + 64));
+  // projector path: the local step with the fused epilogue, the guard on yin
+  // (iterate k - 1; the first one it sees is Y_1, or R_2 of the residual
+  // recurrence), then the projector terms in coefficient space
+  const int first_seen = resw ? 2 : 1;
+  const bool look = k - 1 >= first_seen;
+  int n_part = 0;
+  CHS_TRY(ensure(ctx, im->part, cheb_part_bytes(ctx, n_b)));
+  CHS_TRY(vloc_pipeline(ctx, precision, yin, n_b, yout, mode, yprev, d_coef, 0.0, 0.0,
+                        look ? (double*)im->part.p : nullptr, &n_part, resw, ress));
+  if (look) {
+    hipLaunchKernelGGL(k_norm_guard_prev, dim3(1), dim3(kOneBlock), 0, ctx->stream,
+                       (const double2*)im->part.p, n_part, k - 1, k - 1 == first_seen ? 1 : 0, flag);
+    CHS_LAUNCH_CHECK(ctx);
+  }
+  return cheb_nl_step(ctx, precision, yout, n_b, first, d_coef, resw ? br : nullptr, ress);
+}
+
+// The guard on a projector filter's last iterate y (step k; `first`: it is the
+// only one the guard sees).
+static int cheb_guard_last(chs_context* ctx, int precision, const void* y, int n_b, int k,
+                           bool first, double* flag) {
+  auto* im = ctx->impl;
+  const size_t ne = (size_t)n_b * im->ham.n_pw;
+  CHS_TRY(ensure(ctx, im->part, cheb_part_bytes(ctx, n_b)));
+  // enough workgroups to stream a large block at HBM rate
+  const int blocks = (int)std::min<size_t>(kNormBlocks, (ne + 2047) / 2048);
   if (precision == CHS_C128)
-    hipLaunchKernelGGL((k_sqnorm_part<double>), dim3(kNormBlocks), dim3(kRedThreads), 0,
-                       ctx->stream, (const z64*)yout, ne, (double*)im->part.p);
+    hipLaunchKernelGGL((k_sqnorm_part<double>), dim3(blocks), dim3(kRedThreads), 0, ctx->stream,
+                       (const z64*)y, ne, (double*)im->part.p);
   else
-    hipLaunchKernelGGL((k_sqnorm_part<float>), dim3(kNormBlocks), dim3(kRedThreads), 0,
-                       ctx->stream, (const c32*)yout, ne, (double*)im->part.p);
+    hipLaunchKernelGGL((k_sqnorm_part<float>), dim3(blocks), dim3(kRedThreads), 0, ctx->stream,
+                       (const c32*)y, ne, (double*)im->part.p);
   hipLaunchKernelGGL(k_norm_guard_roll, dim3(1), dim3(256), 0, ctx->stream,
-                     (const double*)im->part.p, kNormBlocks, k, (resw ? guard_first : first) ? 1 : 0,
-                     flag);
+                     (const double*)im->part.p, blocks, k, first ? 1 : 0, flag);
   CHS_LAUNCH_CHECK(ctx);
   return CHS_OK;
 }
@@ -153,6 +214,7 @@ int filter_steps(chs_context* ctx, int precision, void* a, void* b, int n_b, int
     CHS_TRY(cheb_step(ctx, precision, b, n_b, a, a, false, d_coef, k, flag));
     std::swap(a, b);
   }
+  if (H.n_proj > 0) CHS_TRY(cheb_guard_last(ctx, precision, b, n_b, degree, degree == 1, flag));
   *res = b;
   return CHS_OK;
 }
@@ -337,9 +399,10 @@ int chebyshev_filter_res_impl(chs_context* ctx, int precision, const z64* X, int
   }
   for (int k = 1; k < m; ++k) {
     CHS_TRY(cheb_step(ctx, precision, bb, n_b, a, a, false, d_coef, k + 1, flag, Wf,
-                      d_tab + (size_t)k * n_b, br, k == 1));
+                      d_tab + (size_t)k * n_b, br));
     std::swap(a, bb);
   }
+  if (P > 0 && m > 1) CHS_TRY(cheb_guard_last(ctx, precision, bb, n_b, m, m == 2, flag));
   // Y = R_m + X T_m
   if (precision == CHS_C128)
     hipLaunchKernelGGL((k_res_assemble<double>), dim3(ceil_div(ne, 256)), dim3(256), 0, ctx->stream,
@@ -358,48 +421,119 @@ int chebyshev_filter_res_impl(chs_context* ctx, int precision, const z64* X, int
 // coefficients w_x = beta^H x of every Lanczos vector carried along, so a
 // step needs one local H|v>, one beta^H product and one beta product (the
 // Chebyshev step's coefficient-space form):
-//   g = beta^H Hloc v,  y = beta^H H v = g + B D w_v,
-//   c = D w_v - M y  (c = D w_v without S),  S^{-1} H v = Hloc v + beta c,
-//   beta^H S^{-1} H v = g + B c,
+//   g = beta^H Hloc v,  y = Q^{-1} D w_v - g,
+//   c = M y  (c = D w_v without S),  S^{-1} H v = Hloc v + beta c,
+//   beta^H S^{-1} H v = g + B c = g + y - Q^{-1} c  (M (Q^{-1} + B) = 1),
 //   alpha = Re<v|Hloc v> + sum_p D_p |w_v,p|^2,
 //   f = S^{-1} H v - alpha v - beta_{j-1} v_prev (same recurrence on w),
 //   beta_j^2 = <f|f> + sum_p Q_p |w_f,p|^2.
 // B = beta^H beta and M = (Q^{-1} + B)^{-1} are Hermitian, so their rows are
 // read as conjugated columns.
 
-// out[p] = a[p] + s sum_q Mat[p][q] x[q], x[q] = (dx ? dx[q] : 1) xin[q],
-// a[p] = (da ? da[p] : 1) ain[p] (0 without ain); no sum without Mat.
-// One wavefront per row.
-__global__ void __launch_bounds__(256) k_herm_mv(int P, const z64* __restrict__ Mat,
-                                                 const z64* __restrict__ xin,
-                                                 const double* __restrict__ dx,
-                                                 const z64* __restrict__ ain,
-                                                 const double* __restrict__ da, double s,
-                                                 z64* __restrict__ out) {
+// The coefficient-space part of a Lanczos step, one wavefront per row p: with
+// S (Mat = M) c = M y and wu = g + y - Q^{-1} c, y = Q^{-1} D w - g; without
+// (Mat = B) c = D w and wu = g + B c. One launch in place of three dependent
+// matrix-vector products.
+__global__ void __launch_bounds__(256) k_lanczos_coef(int P, const z64* __restrict__ Mat,
+                                                      const z64* __restrict__ w,
+                                                      const z64* __restrict__ g,
+                                                      const double* __restrict__ d,
+                                                      const double* __restrict__ qinv,
+                                                      z64* __restrict__ c, z64* __restrict__ wu) {
   const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (p >= P) return;
+  auto y_of = [&](int q) {
+    const double dq = qinv ? d[q] * qinv[q] : d[q];
+    const z64 wq = w[q];
+    z64 y = mk(dq * wq.x, dq * wq.y);
+    if (qinv) y = y - g[q];
+    return y;
+  };
   double re = 0, im = 0;
-  if (Mat) {
-    const z64* col = Mat + (size_t)p * P;
-    for (int q = lane; q < P; q += 64) {
-      const z64 m = col[q];
-      z64 x = xin[q];
-      if (dx) x = mk(dx[q] * x.x, dx[q] * x.y);
-      re += m.x * x.x + m.y * x.y;  // conj(m) x
-      im += m.x * x.y - m.y * x.x;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-      re += __shfl_down(re, off);
-      im += __shfl_down(im, off);
-    }
+  const z64* col = Mat + (size_t)p * P;  // Hermitian: row p is the conjugate of column p
+  for (int q = lane; q < P; q += 64) {
+    const z64 m = col[q], y = y_of(q);
+    re += m.x * y.x + m.y * y.y;  // conj(m) y
+    im += m.x * y.y - m.y * y.x;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    re += __shfl_down(re, off);
+    im += __shfl_down(im, off);
   }
   if (lane == 0) {
-    z64 a = mk(0.0, 0.0);
-    if (ain) {
-      a = ain[p];
-      if (da) a = mk(da[p] * a.x, da[p] * a.y);
+    const z64 y = y_of(p), gp = g[p];
+    if (qinv) {
+      const double qi = qinv[p];
+      c[p] = mk(re, im);
+      wu[p] = mk(gp.x + y.x - qi * re, gp.y + y.y - qi * im);
+    } else {
+      c[p] = y;
+      wu[p] = mk(gp.x + re, gp.y + im);
     }
-    out[p] = mk(a.x + s * re, a.y + s * im);
+  }
+}
+
+// One-workgroup forms of the Lanczos vector steps for blocks of up to
+// kOneLanczos plane waves, where a launch costs more than the vectors' bytes.
+// alpha_j = Re<v|u> + sum_p D_p |w_v,p|^2 into ab[2 j].
+constexpr int kOneLanczos = 32768;
+
+__global__ void __launch_bounds__(kOneBlock) k_lanczos_alpha(const z64* __restrict__ v,
+                                                             const z64* __restrict__ u, int n,
+                                                             int P, const double* __restrict__ d,
+                                                             const z64* __restrict__ w,
+                                                             double* __restrict__ ab, int j) {
+  __shared__ double sh[17];
+  double a = 0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n; i += kOneBlock) a += v[i].x * u[i].x + v[i].y * u[i].y;
+  for (int p = threadIdx.x; p < P; p += kOneBlock) a += d[p] * norm2(w[p]);
+  const double r = one_block_sum(a, sh);
+  if (threadIdx.x == 0) ab[2 * j] = r;
+}
+
+// f = u - alpha_j v - beta_{j-1} v_prev and the same on the coefficients
+// (j < 0: f and wf are taken as they are), beta = sqrt(<f|f> + sum_p Q_p
+// |w_f,p|^2) into ab[2 slot + 1], then, with `scale`, f and wf divided by it.
+// f: as the last vector's bound only needs beta, it is not scaled then.
+__global__ void __launch_bounds__(kOneBlock) k_lanczos_next(
+    const z64* __restrict__ u, const z64* __restrict__ v, const z64* __restrict__ vp,
+    const z64* __restrict__ wu, const z64* __restrict__ wv, const z64* __restrict__ wvp,
+    double* __restrict__ ab, int j, int slot, int n, int P, const double* __restrict__ Q,
+    int scale, z64* __restrict__ f, z64* __restrict__ wf) {
+  __shared__ double sh[17];
+  const double al = j >= 0 ? ab[2 * j] : 0.0, be = j > 0 ? ab[2 * (j - 1) + 1] : 0.0;
+  double a = 0;
+  // indices n .. n + P - 1 address the coefficient arrays
+  for (int i = threadIdx.x; i < n + P; i += kOneBlock) {
+    const bool pw = i < n;
+    const int q = pw ? i : i - n;
+    z64* dst = pw ? f + q : wf + q;
+    z64 x;
+    if (j >= 0) {
+      const z64 ui = pw ? u[q] : wu[q], vi = pw ? v[q] : wv[q];
+      x = mk(ui.x - al * vi.x, ui.y - al * vi.y);
+      if (j > 0) {
+        const z64 pi = pw ? vp[q] : wvp[q];
+        x = mk(x.x - be * pi.x, x.y - be * pi.y);
+      }
+      *dst = x;
+    } else {
+      x = *dst;
+    }
+    if (pw)
+      a += norm2(x);
+    else if (Q)
+      a += Q[q] * norm2(x);
+  }
+  const double t = one_block_sum(a, sh);
+  const double nb = t > 0 ? sqrt(t) : 0.0;
+  if (threadIdx.x == 0) ab[2 * slot + 1] = nb;
+  if (!scale || !(nb > 0)) return;
+  const double s = 1.0 / nb;
+  for (int i = threadIdx.x; i < n + P; i += kOneBlock) {  // each thread its own elements
+    z64* e = i < n ? f + i : wf + (i - n);
+    *e = mk(e->x * s, e->y * s);
   }
 }
 
@@ -457,11 +591,12 @@ __global__ void k_lanczos_scale(z64* __restrict__ x, z64* __restrict__ wx,
 }
 
 // Extreme eigenvalues of the k x k Lanczos tridiagonal T (alpha_i = ab[2i],
-// beta_i = ab[2i+1]) by bisection on the Sturm count, one thread each;
-// out = {lambda_max(T) + beta_{k-1}, lambda_min(T)}.
-__global__ void k_lanczos_finish(const double* __restrict__ ab, int k, double* __restrict__ out) {
-  const int which = threadIdx.x;  // 0: largest, 1: smallest
-  if (which > 1 || blockIdx.x != 0) return;
+// beta_i = ab[2i+1]) by 64-way multisection on the Sturm count, one wavefront
+// each (bisection by one thread took 59 us); out = {lambda_max(T) + beta_{k-1},
+// lambda_min(T)}.
+__global__ void __launch_bounds__(128) k_lanczos_finish(const double* __restrict__ ab, int k,
+                                                        double* __restrict__ out) {
+  const int which = threadIdx.x >> 6, lane = threadIdx.x & 63;  // 0: largest, 1: smallest
   double gl = INFINITY, gu = -INFINITY, bmax2 = 0.0;
   for (int i = 0; i < k; ++i) {
     const double bl = i > 0 ? fabs(ab[2 * (i - 1) + 1]) : 0.0, br = i + 1 < k ? fabs(ab[2 * i + 1]) : 0.0;
@@ -474,25 +609,29 @@ __global__ void k_lanczos_finish(const double* __restrict__ ab, int k, double* _
   double lo = gl - 4.0 * 2.220446049250313e-16 * tn * k - 2.0 * pivmin;
   double hi = gu + 4.0 * 2.220446049250313e-16 * tn * k + 2.0 * pivmin;
   const int idx = which == 0 ? k - 1 : 0;  // eigenvalue index (ascending)
-  for (int it = 0; it < 200; ++it) {
-    const double mid = 0.5 * (lo + hi);
-    if (mid <= lo || mid >= hi) break;
-    int cnt = 0;  // eigenvalues below mid
-    double q = ab[0] - mid;
+  for (int it = 0; it < 16; ++it) {
+    if (!(hi - lo > 2.220446049250313e-16 * fmax(fabs(lo), fabs(hi)) + 4.0 * pivmin)) break;
+    const double x = lo + (hi - lo) * (double)(lane + 1) / 65.0;
+    int cnt = 0;  // eigenvalues below x
+    double q = ab[0] - x;
     if (fabs(q) < pivmin) q = -pivmin;
     cnt += q < 0.0;
     for (int i = 1; i < k; ++i) {
       const double b = ab[2 * (i - 1) + 1];
-      q = ab[2 * i] - mid - b * b / q;
+      q = ab[2 * i] - x - b * b / q;
       if (fabs(q) < pivmin) q = -pivmin;
       cnt += q < 0.0;
     }
-    if (cnt <= idx) lo = mid;
-    else hi = mid;
+    const int below = __popcll(__ballot(cnt <= idx));  // lanes 0 .. below-1 lie below
+    const double xlo = __shfl(x, below > 0 ? below - 1 : 0), xhi = __shfl(x, below < 64 ? below : 63);
+    if (below > 0) lo = xlo;
+    if (below < 64) hi = xhi;
   }
-  const double lam = 0.5 * (lo + hi);
-  if (which == 0) out[0] = lam + ab[2 * (k - 1) + 1];
-  else out[1] = lam;
+  if (lane == 0) {
+    const double lam = 0.5 * (lo + hi);
+    if (which == 0) out[0] = lam + ab[2 * (k - 1) + 1];
+    else out[1] = lam;
+  }
 }
 
 static int dot_re_into(chs_context* ctx, const z64* a, const z64* b, size_t n, double* dst) {
@@ -551,7 +690,7 @@ int lanczos_impl(chs_context* ctx, int k, uint64_t seed, double* upper, double* 
     im->lanczos_seed = seed;
     im->lanczos_n = n;
   }
-  CHS_TRY(ensure(ctx, im->lin_ws, 4 * vb + 7 * (size_t)std::max(P, 1) * sizeof(z64) +
+  CHS_TRY(ensure(ctx, im->lin_ws, 4 * vb + 6 * (size_t)std::max(P, 1) * sizeof(z64) +
                                       64 * sizeof(double)));
   z64* base = (z64*)im->lin_ws.p;
   // three rotating Lanczos vectors (current, previous, next) and H|v>
@@ -560,73 +699,82 @@ int lanczos_impl(chs_context* ctx, int k, uint64_t seed, double* upper, double* 
   z64* pb = base + 4 * (size_t)n;  // projector coefficients
   const size_t P1 = (size_t)std::max(P, 1);
   z64* wvec[3] = {pb, pb + P1, pb + 2 * P1};
-  z64 *g = pb + 3 * P1, *y = pb + 4 * P1, *c = pb + 5 * P1, *wu = pb + 6 * P1;
-  double* ab = (double*)(pb + 7 * P1);  // alpha/beta pairs + scratch
+  z64 *g = pb + 3 * P1, *c = pb + 4 * P1, *wu = pb + 5 * P1;
+  double* ab = (double*)(pb + 6 * P1);  // alpha/beta pairs + scratch
   double* red = ab + 40;
-  const z64 one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
+  const z64 one_c = mk(1.0, 0.0), zero = mk(0.0, 0.0);
   const z64* beta = (const z64*)H.beta;
   const c32* beta32 = beta_c64 ? (const c32*)H.beta_f.p : nullptr;
   // op(beta) x: op C gives the coefficients beta^H x, op N adds beta c to u
   auto bprod = [&](char op, int m, int kk, const z64* x, z64 bt, z64* yv) -> int {
-    if (beta32) return zgemv_c32(ctx, op, m, kk, one, beta32, n, x, bt, yv);
-    return zgemm(ctx, op, 'N', m, 1, kk, one, beta, n, x, kk, bt, yv, m);
+    if (beta32) return zgemv_c32(ctx, op, m, kk, one_c, beta32, n, x, bt, yv);
+    return zgemm(ctx, op, 'N', m, 1, kk, one_c, beta, n, x, kk, bt, yv, m);
   };
-  const z64* B = (const z64*)H.bmat.p;
-  const z64* M = gen ? (const z64*)H.sinv_m.p : nullptr;
+  const z64* Mat = (const z64*)(gen ? H.sinv_m.p : H.bmat.p);
   const double* Q = gen ? H.qion : nullptr;
+  const double* qinv = gen ? (const double*)H.qinv.p : nullptr;
   const unsigned nblk = (unsigned)ceil_div((size_t)n + P, 256);
+  const bool one = n <= kOneLanczos;  // one-workgroup vector steps
   int cur = 0, prv = 1, nxt = 2;
   CHS_HIP(ctx, hipMemcpyAsync(vec[cur], im->lanczos_v0.p, vb, hipMemcpyDeviceToDevice,
                               ctx->stream));
   CHS_HIP(ctx, hipMemsetAsync(ab, 0, 40 * sizeof(double), ctx->stream));
   // normalise: v /= sqrt(<v|v> + sum Q |w_v|^2)
   if (P > 0) CHS_TRY(bprod('C', P, n, vec[cur], zero, wvec[cur]));
-  CHS_TRY(dot_re_into(ctx, vec[cur], vec[cur], n, red));
-  hipLaunchKernelGGL(k_lanczos_scalar, dim3(1), dim3(256), 0, ctx->stream, P, Q, wvec[cur],
-                     wvec[cur], red, ab, 16, 1);
-  CHS_LAUNCH_CHECK(ctx);
-  hipLaunchKernelGGL(k_lanczos_scale, dim3(nblk), dim3(256), 0, ctx->stream, vec[cur], wvec[cur],
-                     ab, 16, (size_t)n, P);
+  if (one) {
+    hipLaunchKernelGGL(k_lanczos_next, dim3(1), dim3(kOneBlock), 0, ctx->stream, u, u, u, wu, wu,
+                       wu, ab, -1, 16, n, P, Q, 1, vec[cur], wvec[cur]);
+  } else {
+    CHS_TRY(dot_re_into(ctx, vec[cur], vec[cur], n, red));
+    hipLaunchKernelGGL(k_lanczos_scalar, dim3(1), dim3(256), 0, ctx->stream, P, Q, wvec[cur],
+                       wvec[cur], red, ab, 16, 1);
+    hipLaunchKernelGGL(k_lanczos_scale, dim3(nblk), dim3(256), 0, ctx->stream, vec[cur], wvec[cur],
+                       ab, 16, (size_t)n, P);
+  }
   CHS_LAUNCH_CHECK(ctx);
   for (int j = 0; j < k; ++j) {
     CHS_TRY(vloc_pipeline(ctx, CHS_C128, vec[cur], 1, u, EPI_HPSI, nullptr, nullptr, 0, 0, nullptr,
                           nullptr));
-    CHS_TRY(dot_re_into(ctx, vec[cur], u, n, red));
-    hipLaunchKernelGGL(k_lanczos_scalar, dim3(1), dim3(256), 0, ctx->stream, P, H.dion,
-                       wvec[cur], wvec[cur], red, ab, j, 0);
+    if (one) {
+      hipLaunchKernelGGL(k_lanczos_alpha, dim3(1), dim3(kOneBlock), 0, ctx->stream, vec[cur], u, n,
+                         P, H.dion, wvec[cur], ab, j);
+    } else {
+      CHS_TRY(dot_re_into(ctx, vec[cur], u, n, red));
+      hipLaunchKernelGGL(k_lanczos_scalar, dim3(1), dim3(256), 0, ctx->stream, P, H.dion,
+                         wvec[cur], wvec[cur], red, ab, j, 0);
+    }
     CHS_LAUNCH_CHECK(ctx);
     if (P > 0) {
-      const unsigned pblk = (unsigned)ceil_div(P, 4);
       CHS_TRY(bprod('C', P, n, u, zero, g));
-      hipLaunchKernelGGL(k_herm_mv, dim3(pblk), dim3(256), 0, ctx->stream, P, B, wvec[cur],
-                         H.dion, g, nullptr, 1.0, y);
+      hipLaunchKernelGGL(k_lanczos_coef, dim3(ceil_div(P, 4)), dim3(256), 0, ctx->stream, P, Mat,
+                         wvec[cur], g, H.dion, qinv, c, wu);
       CHS_LAUNCH_CHECK(ctx);
-      hipLaunchKernelGGL(k_herm_mv, dim3(pblk), dim3(256), 0, ctx->stream, P, M, y, nullptr,
-                         wvec[cur], H.dion, -1.0, c);
-      CHS_LAUNCH_CHECK(ctx);
-      hipLaunchKernelGGL(k_herm_mv, dim3(pblk), dim3(256), 0, ctx->stream, P, B, c, nullptr, g,
-                         nullptr, 1.0, wu);
-      CHS_LAUNCH_CHECK(ctx);
-      CHS_TRY(bprod('N', n, P, c, one, u));
+      CHS_TRY(bprod('N', n, P, c, one_c, u));
     }
-    hipLaunchKernelGGL(k_lanczos_f, dim3(nblk), dim3(256), 0, ctx->stream, u, vec[cur], vec[prv],
-                       wu, wvec[cur], wvec[prv], ab, j, (size_t)n, P, vec[nxt], wvec[nxt]);
+    const int more = j + 1 < k ? 1 : 0;
+    if (one) {
+      hipLaunchKernelGGL(k_lanczos_next, dim3(1), dim3(kOneBlock), 0, ctx->stream, u, vec[cur],
+                         vec[prv], wu, wvec[cur], wvec[prv], ab, j, j, n, P, Q, more, vec[nxt],
+                         wvec[nxt]);
+    } else {
+      hipLaunchKernelGGL(k_lanczos_f, dim3(nblk), dim3(256), 0, ctx->stream, u, vec[cur], vec[prv],
+                         wu, wvec[cur], wvec[prv], ab, j, (size_t)n, P, vec[nxt], wvec[nxt]);
+      CHS_TRY(dot_re_into(ctx, vec[nxt], vec[nxt], n, red));
+      hipLaunchKernelGGL(k_lanczos_scalar, dim3(1), dim3(256), 0, ctx->stream, P, Q, wvec[nxt],
+                         wvec[nxt], red, ab, j, 1);
+      if (more)
+        hipLaunchKernelGGL(k_lanczos_scale, dim3(nblk), dim3(256), 0, ctx->stream, vec[nxt],
+                           wvec[nxt], ab, j, (size_t)n, P);
+    }
     CHS_LAUNCH_CHECK(ctx);
-    CHS_TRY(dot_re_into(ctx, vec[nxt], vec[nxt], n, red));
-    hipLaunchKernelGGL(k_lanczos_scalar, dim3(1), dim3(256), 0, ctx->stream, P, Q, wvec[nxt],
-                       wvec[nxt], red, ab, j, 1);
-    CHS_LAUNCH_CHECK(ctx);
-    if (j + 1 < k) {
-      hipLaunchKernelGGL(k_lanczos_scale, dim3(nblk), dim3(256), 0, ctx->stream, vec[nxt],
-                         wvec[nxt], ab, j, (size_t)n, P);
-      CHS_LAUNCH_CHECK(ctx);
+    if (more) {
       const int t = prv;
       prv = cur;
       cur = nxt;
       nxt = t;
     }
   }
-  hipLaunchKernelGGL(k_lanczos_finish, dim3(1), dim3(64), 0, ctx->stream, ab, k, red + 4);
+  hipLaunchKernelGGL(k_lanczos_finish, dim3(1), dim3(128), 0, ctx->stream, ab, k, red + 4);
   CHS_LAUNCH_CHECK(ctx);
   double hr[2];
   CHS_HIP(ctx, hipMemcpyAsync(hr, red + 4, 2 * sizeof(double), hipMemcpyDeviceToHost,
