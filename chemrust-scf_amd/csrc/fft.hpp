@@ -147,7 +147,7 @@ CHS_SPLIT(32, 4, 8, 9, 5, 40)     // 48 (ideal 48)
 CHS_SPLIT(36, 4, 9, 10, 4, 41)    // 60 (ideal 52)
 CHS_SPLIT(48, 4, 12, 13, 9, 108)  // 64 (ideal 64)
 CHS_SPLIT(64, 8, 8, 9, 9, 72)     // 64 (ideal 64)
-CHS_SPLIT(72, 8, 9, 12, 10, 105)  // 84 (ideal 68)
+CHS_SPLIT(72, 8, 9, 9, 9, 88)     // 100 (ideal 68; 84 with 12, 10, 105, whose LDS costs a workgroup per CU)
 CHS_SPLIT(96, 8, 12, 15, 9, 140)  // 80 (ideal 80)
 CHS_SPLIT(108, 12, 9, 10, 13, 137)// 126 (ideal 84)
 CHS_SPLIT(128, 8, 16, 17, 9, 144) // 96 (ideal 96)
@@ -804,6 +804,18 @@ __device__ __forceinline__ void row_density(const cplx<T>* crow, slot_t<N, T>* s
   constexpr int R = (N1 + N2 - 1) / N2, PA = RowScratch<N, T>::PA;
   using W = Window<N>;
   using SL = Slot<N, T>;
+  // the row's sums so far, loaded ahead of the transform that hides their
+  // latency (complex64 at 108 points has no registers for two rounds of them)
+  constexpr bool AHEAD = sizeof(T) == 8 || R == 1;
+  double o[R][N2];
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (lane + r * N2 < N1) {
+#pragma unroll
+        for (int k2 = 0; k2 < N2; ++k2) o[r][k2] = orow[lane + r * N2 + N1 * k2];
+      }
+  }
   cplx<T> b[R][N2];
   {
     cplx<T> a[N1];
@@ -847,7 +859,8 @@ __device__ __forceinline__ void row_density(const cplx<T>* crow, slot_t<N, T>* s
 #pragma unroll
       for (int k2 = 0; k2 < N2; ++k2) {
         const double re = (double)b[r][k2].x, im = (double)b[r][k2].y;
-        orow[k1 + N1 * k2] += f * (re * re + im * im);
+        const double so_far = AHEAD ? o[r][k2] : orow[k1 + N1 * k2];
+        orow[k1 + N1 * k2] = so_far + f * (re * re + im * im);
       }
     }
   }

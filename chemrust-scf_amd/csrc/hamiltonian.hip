@@ -102,6 +102,15 @@ struct AccRho {
   }
 };
 
+// Zeros of a compact plane with the window's row stride: only the rows outside
+// the zero window, the ones the inverse y-lines read (they write every row).
+template <int N, typename T> __device__ __forceinline__ void zero_window_plane(cplx<T>* cmp) {
+  using W = Window<N>;
+  constexpr int GAP = (W::HI > W::LO ? W::HI - W::LO : 0) * W::RS, TOP = W::LO * W::RS;
+  for (int i = threadIdx.x; i < N * W::RS - GAP; i += blockDim.x)
+    cmp[GAP > 0 && i >= TOP ? i + GAP : i] = zero_c<T>();
+}
+
 // compact plane <-> one full x row, by the N2 lanes of a group
 template <int N, typename T>
 __device__ __forceinline__ void expand_row(const cplx<T>* cmp_row, cplx<T>* rb, const StickArgs& st,
@@ -129,7 +138,7 @@ __device__ __forceinline__ void expand_row(const cplx<T>* cmp_row, cplx<T>* rb, 
 // the plane). With 8-byte scratch slots in complex128 and the tile pitches of
 // Split<N> the launch went from 5.84 to 4.95 ms (108 points, 512 bands) and
 // from 0.456 to 0.33 ms (72 points, 160 bands); complex64 at 72 points 0.181
-// to 0.165 ms.
+// to 0.15 ms.
 template <int N, typename T, int TPB, bool PR>
 __global__ void __launch_bounds__(TPB) k_plane(cplx<T>* __restrict__ sbuf, StickArgs st,
                                                const T* __restrict__ veff, int nrb, int n_b,
@@ -164,7 +173,10 @@ __global__ void __launch_bounds__(TPB) k_plane(cplx<T>* __restrict__ sbuf, Stick
   constexpr bool PF = sizeof(T) == 4 && TPB <= 512;
   RowV<N, T> vv;
   if (PF && rows) vv.load(vz + (PR ? W::row(g) : g) * N, lane);
-  for (int i = threadIdx.x; i < N * RS; i += blockDim.x) cmp[i] = zero_c<T>();
+  if constexpr (PR)
+    zero_window_plane<N, T>(cmp);
+  else
+    for (int i = threadIdx.x; i < N * RS; i += blockDim.x) cmp[i] = zero_c<T>();
   for (int i = threadIdx.x; i < N; i += blockDim.x) act_of[i] = st.act_of[i];
   if (LT) LaneTw<N>::fill(twl, tw);
   __syncthreads();
@@ -384,7 +396,7 @@ k_density_plane_w(const cplx<T>* __restrict__ sbuf,
     if (f == 0.0) continue;
     const cplx<T>* plane = sbuf + ((size_t)b * N + z) * st.ld;
     __syncthreads();
-    for (int i = threadIdx.x; i < N * RS; i += blockDim.x) cmp[i] = zero_c<T>();
+    zero_window_plane<N, T>(cmp);
     __syncthreads();
     for (int s = threadIdx.x; s < st.n_st; s += blockDim.x) cmp[st.iy[s] * RS + st.act[s]] = plane[s];
     __syncthreads();
@@ -563,6 +575,15 @@ static int plane_launch(chs_context* ctx, int n, const StickArgs& sa, size_t csz
   // kernel loads that row's V_eff ahead of its loop), and a 512-thread
   // workgroup has more groups than a 32- or 36-point plane has rows
   nrb = std::min(nrb, n);
+  // the fewest that keep the rounds over the rows and over the active columns,
+  // where that lets another workgroup onto the CU (complex64 at 72 points, 512
+  // threads: 36 of 56 groups, three workgroups in place of two, 0.191 -> 0.174
+  // ms for 160 bands); otherwise whole wavefronts of groups are better
+  // (complex128 at 72 points: 24 in place of 28 groups cost 4%)
+  const int rr = (n + nrb - 1) / nrb, ry = (sa.n_act + nrb - 1) / nrb;
+  const int few = std::max((n + rr - 1) / rr, (sa.n_act + ry - 1) / ry);
+  auto per_cu = [&](int g) { return lim / (int)(cmp_bytes + (size_t)g * row_bytes + tab_bytes); };
+  if (per_cu(few) > per_cu(nrb)) nrb = few;
   out->nrb = nrb;
   out->threads = threads;
   out->lds = cmp_bytes + (size_t)nrb * row_bytes + tab_bytes;
@@ -733,8 +754,8 @@ int vloc_timed(chs_context* ctx, int precision, const void* psi, int n_b, void* 
 }
 
 // Launch-shape autotuner of the H|psi> pipeline for the bound grid: every
-// (sticks per block, plane-kernel threads, row-buffer divisor) candidate
-// that fits is timed on
+// sticks-per-block and every (plane-kernel threads, row-buffer divisor)
+// candidate that fits is timed on
 // n_b bands at the given precision (HIP events, `reps` runs after one
 // warm-up) and the fastest is kept for (grid, precision).
 int vloc_autotune(chs_context* ctx, int precision, const void* psi, int n_b, void* out, int reps,
@@ -744,24 +765,33 @@ int vloc_autotune(chs_context* ctx, int precision, const void* psi, int n_b, voi
   const size_t csz = precision == CHS_C128 ? 16 : 8;
   auto key = std::make_pair(n, precision);
   VlocTune best{};
-  double best_t = 1e300;
+  // the z passes depend on the sticks per block, the plane kernel on its
+  // threads and divisor: each is tuned by its own kernels' times
+  auto timed = [&](const VlocTune& cand, double* ms) -> int {
+    ctx->impl->vloc_tune[key] = cand;
+    CHS_TRY(vloc_timed(ctx, precision, psi, n_b, out, 1, ms));
+    return vloc_timed(ctx, precision, psi, n_b, out, reps, ms);
+  };
+  double ms[3], best_z = 1e300, best_p = 1e300;
   for (int sb : {16, 32, 64}) {
     if (!sb_fits(n, csz, sb)) continue;
-    for (int threads : {256, 512, 1024})
-      for (int div : {1, 2, 4}) {
-        if (threads == 1024 && csz != 8) continue;
-        const VlocTune cand{sb, div, threads};
-        ctx->impl->vloc_tune[key] = cand;
-        double ms[3];
-        CHS_TRY(vloc_timed(ctx, precision, psi, n_b, out, 1, ms));
-        CHS_TRY(vloc_timed(ctx, precision, psi, n_b, out, reps, ms));
-        const double t = ms[0] + ms[1] + ms[2];
-        if (t < best_t) {
-          best_t = t;
-          best = cand;
-        }
-      }
+    CHS_TRY(timed(VlocTune{sb, 1, 256}, ms));
+    if (ms[0] + ms[2] < best_z) {
+      best_z = ms[0] + ms[2];
+      best.sb = sb;
+    }
   }
+  for (int threads : {256, 512, 1024})
+    for (int div : {1, 2, 4}) {
+      if (threads == 1024 && csz != 8) continue;
+      CHS_TRY(timed(VlocTune{best.sb, div, threads}, ms));
+      if (ms[1] < best_p) {
+        best_p = ms[1];
+        best.nrb_div = div;
+        best.threads = threads;
+      }
+    }
+  const double best_t = best_z + best_p;
   ctx->impl->vloc_tune[key] = best;
   tune_cache_store(ctx, "vloc " + std::to_string(n) + " " + std::to_string(precision) + " " +
                             std::to_string(best.sb) + " " + std::to_string(best.nrb_div) + " " +

@@ -134,7 +134,7 @@ struct GemmKey {
 struct VlocTune {
   int sb = 32;
   int nrb_div = 1;
-  int threads = 256;  // plane kernel workgroup size (256 or 512)
+  int threads = 256;  // plane kernel workgroup size (256 or 512; complex64 also 1024)
 };
 
 }  // namespace chs
