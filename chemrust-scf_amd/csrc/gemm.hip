@@ -141,6 +141,18 @@ template <typename T> struct MfmaTile<T, 3> {
   static constexpr int BM = 64, BN = 64, BK = 32, WTM = 2, WTN = 2;
   static constexpr int WAVES = sizeof(T) == 8 ? 1 : 2;
 };
+// complex64 tiles with fewer padded rows or columns (gemm_variant says when they
+// are tried): 96 x 64 for heights like 864 = 9 x 96, 96 x 32 for widths like
+// 160 = 5 x 32. 864 x 512 x 80,725 (beta^H O) 1.90 -> 1.78 ms, 41,000 x 397 x 864
+// 0.847 -> 0.825 ms, 23,847 x 160 x 256 84 -> 72 us.
+template <> struct MfmaTile<float, 4> {
+  static constexpr int BM = 96, BN = 64, BK = 16, WTM = 3, WTN = 2;
+  static constexpr int WAVES = 3;
+};
+template <> struct MfmaTile<float, 5> {
+  static constexpr int BM = 96, BN = 32, BK = 16, WTM = 3, WTN = 1;
+  static constexpr int WAVES = 4;
+};
 template <> struct MfmaTile<double, 2> {
   static constexpr int BM = 128, BN = 64, BK = 8, WTM = 4, WTN = 2;
   static constexpr int WAVES = 1;
@@ -297,6 +309,12 @@ __attribute__((amdgpu_waves_per_eu(MfmaTile<T, V>::WAVES))) k_gemm_mfma(int m, i
       Bs[kk][c] = rb[j];
     }
   };
+  // Workgroups that share a CU (every 256th or so) get two wave priorities, so
+  // that their product phases do not run in step and leave the matrix cores
+  // idle together (80,725 x 512 x 864 complex64: 1.83 -> 1.79 ms; the 96-row
+  // tiles, three wavefronts per SIMD, lose by it)
+  if constexpr (sizeof(T) == 4 && V == 1 && CL)
+    if ((blockIdx.x >> 8) & 1) __builtin_amdgcn_s_setprio(2);
   auto products = [&]() {
 #pragma unroll
     for (int s = 0; s < BK / 4; ++s) {
@@ -683,6 +701,13 @@ template <typename T>
 static void tile_dims(int variant, int* bm, int* bn, int* bk) {
   *bm = GBM; *bn = GBN; *bk = GBK;
   if (variant == 6) *bm = *bn = *bk = kSM;
+  if (variant == 7 || variant == 8) {
+    using T4 = MfmaTile<float, 4>;
+    using T5 = MfmaTile<float, 5>;
+    *bm = variant == 7 ? T4::BM : T5::BM;
+    *bn = variant == 7 ? T4::BN : T5::BN;
+    *bk = variant == 7 ? T4::BK : T5::BK;
+  }
   if (variant == 1 || variant == 3) {
     *bm = MfmaTile<T, 1>::BM; *bn = MfmaTile<T, 1>::BN; *bk = MfmaTile<T, 1>::BK;
   } else if (variant == 5) {
@@ -741,7 +766,8 @@ static int gemm_launch(chs_context* ctx, int choice, int oa, int ob, int m, int 
   // the offset-addressed kernels (3, 4, 5) only while their offsets fit 32 bits;
   // otherwise the bounds-tested kernel of the same tile
   if (variant == 6 && (oa == 1 || ob != 0 || tri)) variant = 3;
-  if (variant >= 3 && variant <= 5) {
+  if (variant >= 7 && (sizeof(T) == 8 || oa == 1 || ob != 0 || tri)) variant = 3;
+  if (variant >= 3 && variant != 6) {
     int bm0, bn0, bk0;
     tile_dims<T>(variant, &bm0, &bn0, &bk0);
     if (!cl_offsets_fit<T>(oa, ob, m, n, lda, ldb, bk0)) variant = variant == 4 ? 2 : 1;
@@ -766,6 +792,21 @@ static int gemm_launch(chs_context* ctx, int choice, int oa, int ob, int m, int 
     else
       hipLaunchKernelGGL((k_gemm_small<T, 2>), g3, dim3(256), 0, ctx->stream, m, n, k, alpha, A,
                          lda, B, ldb, beta, C, ldc, klen, part);
+  } else if (variant >= 7) {
+    if constexpr (sizeof(T) == 4) {
+#define CHS_GEMM_96(OA, V)                                                                       \
+  hipLaunchKernelGGL((k_gemm_mfma<T, OA, 0, V, true>), g1, dim3(256), 0, ctx->stream, m, n, k,   \
+                     alpha, A, lda, B, ldb, beta, C, ldc, klen, ksplit, nfast, tri, part)
+      if (variant == 7 && oa == 0)
+        CHS_GEMM_96(0, 4);
+      else if (variant == 7)
+        CHS_GEMM_96(2, 4);
+      else if (oa == 0)
+        CHS_GEMM_96(0, 5);
+      else
+        CHS_GEMM_96(2, 5);
+#undef CHS_GEMM_96
+    }
   } else {
 #define CHS_GEMM_CASE(OA, OB)                                                                    \
   if (oa == OA && ob == OB) {                                                                    \
@@ -802,6 +843,11 @@ static int gemm_launch(chs_context* ctx, int choice, int oa, int ob, int m, int 
   return CHS_OK;
 }
 
+// longest K slice of a complex64 product: beta^H O of the 216-atom cell in 7
+// slices of 11,536 (1.77 ms) put the filter's error at 4.7e-7 of the result, in
+// 28 of 2,896 (1.80 ms) at 3.7e-7
+constexpr int kMaxChain = 6144;
+
 // most 32 x 32 tiles the small-product kernel is tried with: four workgroups per
 // CU (with more, 64 x 64 tiles fill the chip and share operands through LDS: at
 // 3,730 tiles of the 64-atom O + beta C both take 86 us)
@@ -812,8 +858,9 @@ constexpr double kSmallWork = 4e9;
 
 // Kernel choice for a GEMM shape: variant (low 4 bits: 0 vector-FMA 64 x 64,
 // 1 MFMA 64 x 64, 2 MFMA 128-wide, 3 and 4 the same with clamped loads, 5
-// MFMA 64 x 64 x 32 with clamped loads, 6 the small-product kernel) and
-// split-K target (bits 4-5, index into kSplitTargets). The small-product kernel
+// MFMA 64 x 64 x 32 with clamped loads, 6 the small-product kernel, 7 and 8
+// complex64 MFMA 96 x 64 and 96 x 32) and split-K target (bits 4-5, index into
+// kSplitTargets). The small-product kernel
 // is a candidate for op(A) in {N, C}, B not transposed and up to kSmallTiles
 // tiles and kSmallWork products, in complex64 and, where the caller asks (`small`), in complex128: the
 // FP64 products of Rayleigh-Ritz keep their summation order. Chosen once per (precision, ops, m, n, k) by timing every
@@ -851,11 +898,21 @@ static int gemm_variant(chs_context* ctx, int oa, int ob, int m, int n, int k, c
   const bool sm = (small || sizeof(T) == 4) && oa != 1 && ob == 0 && !tri &&
                   (int)(ceil_div(m, kSM) * ceil_div(n, kSM)) <= kSmallTiles &&
                   (double)m * n * k <= kSmallWork;
-  for (int v = big ? 1 : 0; v < (sm ? 7 : 6); ++v) {
+  const bool c64nn = sizeof(T) == 4 && oa != 1 && ob == 0 && !tri;
+  auto padded = [](int x, int tile) { return (x + tile - 1) / tile * tile; };
+  for (int v = big ? 1 : 0; v < 9; ++v) {
+    if (v == 6 && !sm) continue;
+    // 96-row tiles where they pad the rows no more than 64-row ones, 32-column
+    // tiles where they pad the columns less
+    if (v == 7 && !(c64nn && big && padded(m, 96) <= padded(m, 64))) continue;
+    if (v == 8 && !(c64nn && padded(n, 32) < padded(n, 64))) continue;
     int prev_split = -1;
     for (int ti = 0; ti < kNumSplitTargets; ++ti) {
       int ks, kl;
       variant_plan<T>(v, m, n, k, kSplitTargets[ti], tri, &ks, &kl);
+      // complex64 sums run at most kMaxChain products before the slices are
+      // added, unless no target cuts K that far
+      if (sizeof(T) == 4 && kl > kMaxChain && ti + 1 < kNumSplitTargets) continue;
       if (ks == prev_split) continue;  // same launch as a smaller target
       prev_split = ks;
       const int c = v | (ti << 4);
