@@ -424,24 +424,25 @@ k_mlp_pass(const unsigned short* __restrict__ wbf, const float* __restrict__ fea
 __global__ void __launch_bounds__(64) k_mlp_band_sums(const double* __restrict__ tsum, int nbb,
                                                       int tpb, double* __restrict__ bcoef,
                                                       double* __restrict__ lossv) {
-  const int j = blockIdx.x;
-  double A = 0, B = 0, E = 0;
-  for (int t = threadIdx.x; t < tpb; t += 64) {
-    const double* p = tsum + 3 * ((size_t)j * tpb + t);
-    A += p[0];
-    B += p[1];
-    E += p[2];
+  for (int j = blockIdx.x; j < nbb; j += gridDim.x) {
+    double A = 0, B = 0, E = 0;
+    for (int t = threadIdx.x; t < tpb; t += 64) {
+      const double* p = tsum + 3 * ((size_t)j * tpb + t);
+      A += p[0];
+      B += p[1];
+      E += p[2];
+    }
+    for (int k = 32; k > 0; k >>= 1) {
+      A += __shfl_xor(A, k);
+      B += __shfl_xor(B, k);
+      E += __shfl_xor(E, k);
+    }
+    if (threadIdx.x != 0) continue;
+    const bool used = B > 0.0 && E > 0.0;
+    bcoef[2 * j] = used ? 2.0 * A / (B * E) / nbb : 0.0;
+    bcoef[2 * j + 1] = used ? A / B : 0.0;
+    lossv[j] = used ? (1.0 - A * A / (B * E)) / nbb : 0.0;
   }
-  for (int k = 32; k > 0; k >>= 1) {
-    A += __shfl_xor(A, k);
-    B += __shfl_xor(B, k);
-    E += __shfl_xor(E, k);
-  }
-  if (threadIdx.x != 0) return;
-  const bool used = B > 0.0 && E > 0.0;
-  bcoef[2 * j] = used ? 2.0 * A / (B * E) / nbb : 0.0;
-  bcoef[2 * j + 1] = used ? A / B : 0.0;
-  lossv[j] = used ? (1.0 - A * A / (B * E)) / nbb : 0.0;
 }
 
 // Gradient from the block partials, 16 parameters per workgroup with 16
@@ -673,7 +674,7 @@ static int mlp_batch(chs_context* ctx, chs_mlp* m, const float* feat, const floa
   hipLaunchKernelGGL(k_mlp_pass<0>, dim3(nblk0), dim3(64 * kMlpWaves), 0, ctx->stream, wbf, feat, r,
                      e, w, NB, Lb, nbb, off, stride, (double*)m->tsum.p, (const double*)nullptr,
                      (float*)nullptr);
-  hipLaunchKernelGGL(k_mlp_band_sums, dim3(nbb), dim3(64), 0, ctx->stream,
+  hipLaunchKernelGGL(k_mlp_band_sums, dim3(std::min(nbb, 1 << 20)), dim3(64), 0, ctx->stream,
                      (const double*)m->tsum.p, nbb, tpb, bcoef, lossv);
   hipLaunchKernelGGL(k_mlp_pass<1>, dim3(nblk1), dim3(64 * kMlpWaves), 0, ctx->stream, wbf, feat, r,
                      e, w, NB, Lb, nbb, off, stride, (double*)nullptr, (const double*)bcoef,

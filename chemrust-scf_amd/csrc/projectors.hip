@@ -790,10 +790,11 @@ int chs_bind_projectors(chs_context* ctx, int n_proj, const double* d_beta, cons
   CHS_TRY(zgemm(ctx, 'C', 'N', P, P, H.n_pw, mk(1.0, 0.0), (const z64*)d_beta, H.n_pw,
                 (const z64*)d_beta, H.n_pw, mk(0.0, 0.0), (z64*)H.bmat.p, P));
   CHS_TRY(hermitise(ctx, (z64*)H.bmat.p, P));
+  // B alone until M exists: a binding whose Cholesky fails keeps S = 1
   CHS_TRY(ensure(ctx, H.kstack, (any ? 2 : 1) * pp * sizeof(z64)));
+  CHS_HIP(ctx, hipMemcpyAsync(H.kstack.p, H.bmat.p, pp * sizeof(z64), hipMemcpyDeviceToDevice,
+                              ctx->stream));
   if (!any) {
-    CHS_HIP(ctx, hipMemcpyAsync(H.kstack.p, H.bmat.p, pp * sizeof(z64), hipMemcpyDeviceToDevice,
-                                ctx->stream));
     CHS_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return CHS_OK;
   }
