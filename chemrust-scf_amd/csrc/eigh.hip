@@ -830,7 +830,9 @@ int heev_tridiag(chs_context* ctx, z64* A, int n, double* w, z64* U) {
   hipLaunchKernelGGL(k_tri_to_complex, dim3(ceil_div((size_t)n * n, 256)), dim3(256), 0,
                      ctx->stream, ws.zt, n, U);
   CHS_LAUNCH_CHECK(ctx);
-  // 3. U <- Q U, blocks of reflectors from the last to the first
+  // 3. U <- Q U, blocks of reflectors from the last to the first (32-wide
+  // products: 64 x 64 tiles keep one to eight workgroups busy, the small-product
+  // kernel up to 80; 160-band Rayleigh-Ritz 3.00 -> 2.93 ms)
   const z64 one = mk(1.0, 0.0), zero = mk(0.0, 0.0), mone = mk(-1.0, 0.0);
   const int nref = n - 1;
   for (int kb = ((nref - 1) / kWY) * kWY; nref > 0 && kb >= 0; kb -= kWY) {
@@ -838,13 +840,13 @@ int heev_tridiag(chs_context* ctx, z64* A, int n, double* w, z64* U) {
     const int rows = n - kb - 1;
     const z64* V = ws.vst + (size_t)kb * n + (kb + 1);
     // V^H V into w2 (free until the T w1 product below)
-    CHS_TRY(zgemm(ctx, 'C', 'N', b, b, rows, one, V, n, V, n, zero, ws.w2, b));
+    CHS_TRY(zgemm_small(ctx, 'C', 'N', b, b, rows, one, V, n, V, n, zero, ws.w2, b));
     hipLaunchKernelGGL(k_wy_tmat, dim3(1), dim3(256), 0, ctx->stream, ws.w2, kb, b, ws.tau,
                        ws.tmat);
     CHS_LAUNCH_CHECK(ctx);
-    CHS_TRY(zgemm(ctx, 'C', 'N', b, n, rows, one, V, n, U + (kb + 1), n, zero, ws.w1, b));
-    CHS_TRY(zgemm(ctx, 'N', 'N', b, n, b, one, ws.tmat, b, ws.w1, b, zero, ws.w2, b));
-    CHS_TRY(zgemm(ctx, 'N', 'N', rows, n, b, mone, V, n, ws.w2, b, one, U + (kb + 1), n));
+    CHS_TRY(zgemm_small(ctx, 'C', 'N', b, n, rows, one, V, n, U + (kb + 1), n, zero, ws.w1, b));
+    CHS_TRY(zgemm_small(ctx, 'N', 'N', b, n, b, one, ws.tmat, b, ws.w1, b, zero, ws.w2, b));
+    CHS_TRY(zgemm_small(ctx, 'N', 'N', rows, n, b, mone, V, n, ws.w2, b, one, U + (kb + 1), n));
   }
   return CHS_OK;
 }

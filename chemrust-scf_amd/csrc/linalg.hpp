@@ -11,7 +11,8 @@ int zgemm(chs_context* ctx, char opa, char opb, int m, int n, int k, z64 alpha, 
 int zgemm_herm(chs_context* ctx, int n, int k, const z64* A, int lda, const z64* B, int ldb, z64* C,
                int ldc);
 // zgemm with the small-product kernel among the tuner's candidates (the
-// filter's products; zgemm itself keeps its kernels and their sums' order).
+// filter's products, the eigensolver's back-transformation; zgemm itself keeps
+// its kernels and their sums' order).
 int zgemm_small(chs_context* ctx, char opa, char opb, int m, int n, int k, z64 alpha, const z64* A,
                 int lda, const z64* B, int ldb, z64 beta, z64* C, int ldc);
 int cgemm(chs_context* ctx, char opa, char opb, int m, int n, int k, c32 alpha, const c32* A,
