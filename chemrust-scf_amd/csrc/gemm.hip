@@ -846,7 +846,7 @@ static int gemm_launch(chs_context* ctx, int choice, int oa, int ob, int m, int 
 // longest K slice of a complex64 product: beta^H O of the 216-atom cell in 7
 // slices of 11,536 (1.77 ms) put the filter's error at 4.7e-7 of the result, in
 // 28 of 2,896 (1.80 ms) at 3.7e-7
-constexpr int kMaxChain = 6144;
+constexpr int kMaxChain = 3072;
 
 // most 32 x 32 tiles the small-product kernel is tried with: four workgroups per
 // CU (with more, 64 x 64 tiles fill the chip and share operands through LDS: at
