@@ -856,14 +856,43 @@ constexpr int kSmallTiles = 1024;
 // tiles' time; 256 x 160 x 23,847 = 9.8e8 is 20% faster)
 constexpr double kSmallWork = 4e9;
 
+// Split-K target of a complex128 product, by its shape alone. The order of its
+// sums, hence the last bits of H_sub and S_sub, sets the signs of Rayleigh-Ritz's
+// eigenvectors (inverse iteration keeps the sign of a rounding error), so it must
+// not follow the tuner's timings: candidates 1% apart (864 x 512 x 80,725: 36
+// slices 3.53 ms, 18 slices 3.57 ms) were picked differently from one context to
+// the next. The smallest target with at least kMinSlices slices (kMinSlicesTri
+// where only the upper tiles are computed), as long as slices stay kMinSlice
+// long: fewer leave part of the chip waiting for the last workgroups (512 x 512
+// upper tiles of K = 80,725: 28 slices 1.70 ms, 56 1.57 ms; 864 x 360 x 63,077:
+// 12 slices 2.11 ms, 24 2.07 ms), shorter ones pay for their partial sums (256 x
+// 256 x 20,815: 32 slices 0.162 ms, 62 0.176 ms; 864 x 864 x 864: 2 slices 0.103
+// ms, 4 0.117 ms). Over 60 shapes of the 64- and 216-atom cells it takes the
+// fastest split or one within 1.5%, but for the upper tiles of 257 to 384 bands
+// (up to 5%).
+constexpr int kMinSlices = 24, kMinSlicesTri = 48, kMinSlice = 512;
+
+static int fixed_split_target(int m, int n, int k, bool tri) {
+  int ks, kl, ti = 0;
+  variant_plan<double>(3, m, n, k, kSplitTargets[0], tri, &ks, &kl);
+  while (ks < (tri ? kMinSlicesTri : kMinSlices) && ti + 1 < kNumSplitTargets) {
+    variant_plan<double>(3, m, n, k, kSplitTargets[ti + 1], tri, &ks, &kl);
+    if (kl < kMinSlice) break;
+    ++ti;
+  }
+  return ti;
+}
+
 // Kernel choice for a GEMM shape: variant (low 4 bits: 0 vector-FMA 64 x 64,
 // 1 MFMA 64 x 64, 2 MFMA 128-wide, 3 and 4 the same with clamped loads, 5
 // MFMA 64 x 64 x 32 with clamped loads, 6 the small-product kernel, 7 and 8
 // complex64 MFMA 96 x 64 and 96 x 32) and split-K target (bits 4-5, index into
 // kSplitTargets). The small-product kernel
 // is a candidate for op(A) in {N, C}, B not transposed and up to kSmallTiles
-// tiles and kSmallWork products, in complex64 and, where the caller asks (`small`), in complex128: the
-// FP64 products of Rayleigh-Ritz keep their summation order. Chosen once per (precision, ops, m, n, k) by timing every
+// tiles and kSmallWork products, in complex64 and, where the caller asks (`small`), in complex128.
+// Every other complex128 product has the split of fixed_split_target, and only
+// the MFMA kernels that cut K into the same slices (and so add in the same order)
+// are candidates. Chosen once per (precision, ops, m, n, k) by timing every
 // distinct launch into a scratch output (HIP events, context stream);
 // outside a stream capture only, otherwise the MFMA 64 x 64 default.
 template <typename T>
@@ -885,7 +914,11 @@ static int gemm_variant(chs_context* ctx, int oa, int ob, int m, int n, int k, c
     *choice = it->second;
     return CHS_OK;
   }
-  *choice = 1;
+  const bool fixed = sizeof(T) == 8 && !small;
+  const int fixed_ti = fixed ? fixed_split_target(m, n, k, tri != 0) : 0;
+  *choice = 1 | (fixed_ti << 4);
+  int fixed_ks = 0, fixed_kl = 0;
+  if (fixed) variant_plan<T>(1, m, n, k, kSplitTargets[fixed_ti], tri, &fixed_ks, &fixed_kl);
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   CHS_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cs));
   if (cs != hipStreamCaptureStatusNone || !im->gemm_autotune) return CHS_OK;
@@ -900,7 +933,7 @@ static int gemm_variant(chs_context* ctx, int oa, int ob, int m, int n, int k, c
                   (double)m * n * k <= kSmallWork;
   const bool c64nn = sizeof(T) == 4 && oa != 1 && ob == 0 && !tri;
   auto padded = [](int x, int tile) { return (x + tile - 1) / tile * tile; };
-  for (int v = big ? 1 : 0; v < 9; ++v) {
+  for (int v = big || fixed ? 1 : 0; v < 9; ++v) {
     if (v == 6 && !sm) continue;
     // 96-row tiles where they pad the rows no more than 64-row ones, 32-column
     // tiles where they pad the columns less
@@ -910,6 +943,7 @@ static int gemm_variant(chs_context* ctx, int oa, int ob, int m, int n, int k, c
     for (int ti = 0; ti < kNumSplitTargets; ++ti) {
       int ks, kl;
       variant_plan<T>(v, m, n, k, kSplitTargets[ti], tri, &ks, &kl);
+      if (fixed && (ti != fixed_ti || ks != fixed_ks || (ks > 1 && kl != fixed_kl))) continue;
       // complex64 sums run at most kMaxChain products before the slices are
       // added, unless no target cuts K that far
       if (sizeof(T) == 4 && kl > kMaxChain && ti + 1 < kNumSplitTargets) continue;
@@ -930,10 +964,7 @@ static int gemm_variant(chs_context* ctx, int oa, int ob, int m, int n, int k, c
         float tr = 0;
         CHS_HIP(ctx, hipEventElapsedTime(&tr, im->ev0, im->ev1));
         t = std::min(t, tr);
-        // far behind: not timed again (complex64 and `small`; other complex128
-        // choices stay as repeatable as three timings make them: the signs of
-        // Rayleigh-Ritz's eigenvectors follow their sums' last bits)
-        if ((sizeof(T) == 4 || small) && t > 1.25 * best) break;
+        if (t > 1.25 * best) break;  // far behind: not timed again
       }
       if (t < best) {
         best = t;
