@@ -62,9 +62,9 @@ struct Hamiltonian {
   DevBuf sinv_m;                 // c128 P x P (Q^-1 + beta^H beta)^-1
   DevBuf sinv_m_f;               // c64 copy
   DevBuf bmat;                   // c128 P x P beta^H beta
-  // left factor of the filter's coefficient step: [M; B M] (2P x P) with S,
-  // B (P x P) without, c128 and c64, and the P reciprocals 1/Q
-  DevBuf kstack, kstack_f, qinv;
+  // left factor of the filter's coefficient step: [N; B N] (2P x P, N =
+  // M Q^{-1}) with S, B (P x P) without, c128 and c64, and a copy of Q
+  DevBuf kstack, kstack_f, qd;
   // projector coefficients carried through a Chebyshev filter (nl_ws: three
   // 2P x n_b slots [step coefficients; W] and a P x n_b one): the slots of
   // W_{k-1}, W_k and G = beta^H O
@@ -78,7 +78,7 @@ struct Hamiltonian {
 };
 
 inline void release_hamiltonian(Hamiltonian& h) {
-  for (DevBuf* b : {&h.veff_f, &h.st_mem, &h.beta_f, &h.sinv_m, &h.sinv_m_f, &h.bmat, &h.kstack, &h.kstack_f, &h.qinv,
+  for (DevBuf* b : {&h.veff_f, &h.st_mem, &h.beta_f, &h.sinv_m, &h.sinv_m_f, &h.bmat, &h.kstack, &h.kstack_f, &h.qd,
                     &h.nl_ws, &h.fscr, &h.h3_cn.buf, &h.h3_nn.buf, &h.h3_exp})
     release(*b);
   h = Hamiltonian{};

@@ -421,55 +421,56 @@ int chebyshev_filter_res_impl(chs_context* ctx, int precision, const z64* X, int
 // coefficients w_x = beta^H x of every Lanczos vector carried along, so a
 // step needs one local H|v>, one beta^H product and one beta product (the
 // Chebyshev step's coefficient-space form):
-//   g = beta^H Hloc v,  y = Q^{-1} D w_v - g,
-//   c = M y  (c = D w_v without S),  S^{-1} H v = Hloc v + beta c,
-//   beta^H S^{-1} H v = g + B c = g + y - Q^{-1} c  (M (Q^{-1} + B) = 1),
+//   g = beta^H Hloc v,  y = D w_v - Q g,
+//   c = M Q^{-1} y  (c = D w_v without S),  S^{-1} H v = Hloc v + beta c,
+//   beta^H S^{-1} H v = g + B c = g + (B N) y,  N = M Q^{-1} = (1 + Q B)^{-1},
 //   alpha = Re<v|Hloc v> + sum_p D_p |w_v,p|^2,
 //   f = S^{-1} H v - alpha v - beta_{j-1} v_prev (same recurrence on w),
 //   beta_j^2 = <f|f> + sum_p Q_p |w_f,p|^2.
-// B = beta^H beta and M = (Q^{-1} + B)^{-1} are Hermitian, so their rows are
-// read as conjugated columns.
+// B = beta^H beta, M = (Q^{-1} + B)^{-1} and B N = (B^{-1} + Q)^{-1} are
+// Hermitian, so their rows are read as conjugated columns.
 
 // The coefficient-space part of a Lanczos step, one wavefront per row p: with
-// S (Mat = M) c = M y and wu = g + y - Q^{-1} c, y = Q^{-1} D w - g; without
-// (Mat = B) c = D w and wu = g + B c. One launch in place of three dependent
-// matrix-vector products.
-__global__ void __launch_bounds__(256) k_lanczos_coef(int P, const z64* __restrict__ Mat,
+// S (M given, KB = B N) y = D w - Q g, c = M Q^{-1} y and wu = g + KB y;
+// without (KB = B) c = y = D w and wu = g + KB y. KB has leading dimension ldk.
+// One launch in place of three dependent matrix-vector products. (g + D w / Q -
+// g - c / Q in place of g + KB y would need no second matrix, and lose eps / (Q B).)
+__global__ void __launch_bounds__(256) k_lanczos_coef(int P, const z64* __restrict__ M,
+                                                      const z64* __restrict__ KB, int ldk,
                                                       const z64* __restrict__ w,
                                                       const z64* __restrict__ g,
                                                       const double* __restrict__ d,
-                                                      const double* __restrict__ qinv,
+                                                      const double* __restrict__ qd,
                                                       z64* __restrict__ c, z64* __restrict__ wu) {
   const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (p >= P) return;
   auto y_of = [&](int q) {
-    const double dq = qinv ? d[q] * qinv[q] : d[q];
-    const z64 wq = w[q];
-    z64 y = mk(dq * wq.x, dq * wq.y);
-    if (qinv) y = y - g[q];
+    z64 y = mk(d[q] * w[q].x, d[q] * w[q].y);
+    if (M) y = mk(y.x - qd[q] * g[q].x, y.y - qd[q] * g[q].y);
     return y;
   };
-  double re = 0, im = 0;
-  const z64* col = Mat + (size_t)p * P;  // Hermitian: row p is the conjugate of column p
+  double re = 0, im = 0, cre = 0, cim = 0;
+  // Hermitian: row p is the conjugate of column p
+  const z64 *kcol = KB + (size_t)p * ldk, *mcol = M ? M + (size_t)p * P : nullptr;
   for (int q = lane; q < P; q += 64) {
-    const z64 m = col[q], y = y_of(q);
-    re += m.x * y.x + m.y * y.y;  // conj(m) y
-    im += m.x * y.y - m.y * y.x;
+    const z64 k = kcol[q], y = y_of(q);
+    re += k.x * y.x + k.y * y.y;  // conj(k) y
+    im += k.x * y.y - k.y * y.x;
+    if (M) {
+      const z64 m = mcol[q], x = mk(y.x / qd[q], y.y / qd[q]);
+      cre += m.x * x.x + m.y * x.y;
+      cim += m.x * x.y - m.y * x.x;
+    }
   }
   for (int off = 32; off > 0; off >>= 1) {
     re += __shfl_down(re, off);
     im += __shfl_down(im, off);
+    cre += __shfl_down(cre, off);
+    cim += __shfl_down(cim, off);
   }
   if (lane == 0) {
-    const z64 y = y_of(p), gp = g[p];
-    if (qinv) {
-      const double qi = qinv[p];
-      c[p] = mk(re, im);
-      wu[p] = mk(gp.x + y.x - qi * re, gp.y + y.y - qi * im);
-    } else {
-      c[p] = y;
-      wu[p] = mk(gp.x + re, gp.y + im);
-    }
+    c[p] = M ? mk(cre, cim) : y_of(p);
+    wu[p] = mk(g[p].x + re, g[p].y + im);
   }
 }
 
@@ -710,9 +711,10 @@ int lanczos_impl(chs_context* ctx, int k, uint64_t seed, double* upper, double* 
     if (beta32) return zgemv_c32(ctx, op, m, kk, one_c, beta32, n, x, bt, yv);
     return zgemm(ctx, op, 'N', m, 1, kk, one_c, beta, n, x, kk, bt, yv, m);
   };
-  const z64* Mat = (const z64*)(gen ? H.sinv_m.p : H.bmat.p);
+  const z64* M = gen ? (const z64*)H.sinv_m.p : nullptr;
+  const z64* KB = gen ? (const z64*)H.kstack.p + P : (const z64*)H.bmat.p;
   const double* Q = gen ? H.qion : nullptr;
-  const double* qinv = gen ? (const double*)H.qinv.p : nullptr;
+  const double* qd = gen ? (const double*)H.qd.p : nullptr;
   const unsigned nblk = (unsigned)ceil_div((size_t)n + P, 256);
   const bool one = n <= kOneLanczos;  // one-workgroup vector steps
   int cur = 0, prv = 1, nxt = 2;
@@ -746,8 +748,8 @@ int lanczos_impl(chs_context* ctx, int k, uint64_t seed, double* upper, double* 
     CHS_LAUNCH_CHECK(ctx);
     if (P > 0) {
       CHS_TRY(bprod('C', P, n, u, zero, g));
-      hipLaunchKernelGGL(k_lanczos_coef, dim3(ceil_div(P, 4)), dim3(256), 0, ctx->stream, P, Mat,
-                         wvec[cur], g, H.dion, qinv, c, wu);
+      hipLaunchKernelGGL(k_lanczos_coef, dim3(ceil_div(P, 4)), dim3(256), 0, ctx->stream, P, M, KB,
+                         gen ? 2 * P : P, wvec[cur], g, H.dion, qd, c, wu);
       CHS_LAUNCH_CHECK(ctx);
       CHS_TRY(bprod('N', n, P, c, one_c, u));
     }

@@ -44,18 +44,17 @@ __global__ void k_diag_add_inv(z64* __restrict__ a, const double* __restrict__ q
   if (i < P) a[(size_t)i + (size_t)i * P].x += 1.0 / q[i];
 }
 
-// [M; B M] (2P x P) and 1/Q, with B M = 1 - Q^{-1} M (M (Q^{-1} + B) = 1).
-__global__ void k_stack_m(const z64* __restrict__ M, const double* __restrict__ q, int P,
-                          z64* __restrict__ K, double* __restrict__ qinv) {
+// N = M Q^{-1} = (1 + Q B)^{-1} into the upper half of the 2P x P stack [N; B N],
+// and a copy of Q. N stays of order one for every Q; Q^{-1} enters by this
+// column scaling alone, so a small Q cancels nothing.
+__global__ void k_stack_n(const z64* __restrict__ M, const double* __restrict__ q, int P,
+                          z64* __restrict__ K, double* __restrict__ qd) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (size_t)P * P) return;
   const int r = (int)(i % P), c = (int)(i / P);
   const z64 v = M[i];
-  const double qi = 1.0 / q[r];
-  z64* col = K + (size_t)c * 2 * P;
-  col[r] = v;
-  col[P + r] = mk((r == c ? 1.0 : 0.0) - qi * v.x, -qi * v.y);
-  if (c == 0) qinv[r] = qi;
+  K[(size_t)c * 2 * P + r] = mk(v.x / q[c], v.y / q[c]);
+  if (r == 0) qd[c] = q[c];
 }
 
 template <typename A, typename B>
@@ -140,14 +139,17 @@ static int nonlocal_t(chs_context* ctx, const cplx<T>* psi, int n_b, cplx<T>* hp
 // O is the local-potential step (the fused H|psi> pipeline's Chebyshev
 // epilogue) and
 //   C = D W_k - M (Z + B D W_k),   Z = beta^H H_loc X_k,
-// B = beta^H beta, M = (Q^{-1} + B)^{-1} (C = D W_k when S = 1). Since
-// M (Q^{-1} + B) = 1 this is C = M y with y = Q^{-1} D W_k - Z. Z follows
-// from G = beta^H O: Z = (e/2)(G + W_{k-1}) + c W_k (first step:
-// Z = e G + c W_0), and W_{k+1} = G + f B C = G + f (B M) y. Two n_pw-long
-// GEMMs per step (G and the beta C update) and one product [M; B M] (f y) into
+// B = beta^H beta, M = (Q^{-1} + B)^{-1} (C = D W_k when S = 1). With
+// N = M Q^{-1} = (1 + Q B)^{-1} = 1 - M B this is C = N y, y = D W_k - Q Z. Z
+// follows from G = beta^H O: Z = (e/2)(G + W_{k-1}) + c W_k (first step:
+// Z = e G + c W_0), and W_{k+1} = G + f B C = G + f (B N) y. Two n_pw-long
+// GEMMs per step (G and the beta C update) and one product [N; B N] (f y) into
 // [f C; W_{k+1}], whose lower half holds G (without S: B (f D W_k) into the
-// lower half). Three dependent P x P products and a scaling pass were a sixth
-// of the k-point set's filter (64 atoms: 26 us each, 12 workgroups).
+// lower half). B N is formed as a product once: taken from M (Q^{-1} + B) = 1 as
+// 1 - Q^{-1} M it loses eps / (Q B) of W_{k+1} (P = 37, degree 12: 1e-11 of the
+// filtered block at Q = 1e-6, 5e-6 at 1e-12; formed so, 5e-16 at each). Three
+// dependent P x P products and a scaling pass were a sixth of the k-point set's
+// filter (64 atoms: 26 us each, 12 workgroups).
 // ---------------------------------------------------------------------------
 // Elementwise part, coef = {c, inv_e} on the device (graph-replayable). W, Wp
 // and G are the lower halves of 2P x n_b slots (leading dimension 2P), `top`
@@ -158,7 +160,7 @@ static int nonlocal_t(chs_context* ctx, const cplx<T>* psi, int n_b, cplx<T>* hp
 template <typename T>
 __global__ void k_cheb_coef(const cplx<T>* __restrict__ G, const cplx<T>* __restrict__ Wp,
                             const cplx<T>* __restrict__ W, const double* __restrict__ d,
-                            const double* __restrict__ qinv, const double* __restrict__ coef,
+                            const double* __restrict__ qd, const double* __restrict__ coef,
                             int first, int P, size_t n, cplx<T>* __restrict__ y,
                             cplx<T>* __restrict__ top, const cplx<T>* __restrict__ BR,
                             const double* __restrict__ ress) {
@@ -182,8 +184,9 @@ __global__ void k_cheb_coef(const cplx<T>* __restrict__ G, const cplx<T>* __rest
     const double sb = ress[b];
     g = mk(g.x - sb * BR[i].x, g.y - sb * BR[i].y);
   }
-  const double e = d[p] * qinv[p] - c;  // Q^{-1} D W - c W
-  y[i] = mk((T)(f * (e * w.x - a1 * g.x - a2 * wp.x)), (T)(f * (e * w.y - a1 * g.y - a2 * wp.y)));
+  const double qp = qd[p], e = d[p] - qp * c;  // D W - c Q W
+  y[i] = mk((T)(f * (e * w.x - qp * (a1 * g.x + a2 * wp.x))),
+            (T)(f * (e * w.y - qp * (a1 * g.y + a2 * wp.y))));
   top[q] = mk((T)0, (T)0);
 }
 
@@ -267,10 +270,10 @@ static int cheb_nl_step_t(chs_context* ctx, cplx<T>* O, int n_b, bool first, con
   if (!h3) CHS_TRY(gemm_filter<T>(ctx, 'C', P, n_b, n_pw, beta, n_pw, O, n_pw, 0.0, G, 2 * P));
   hipLaunchKernelGGL((k_cheb_coef<T>), dim3(ceil_div(pb, 256)), dim3(256), 0, ctx->stream, G,
                      nl_low<T>(H, n_b, H.nl_wp), nl_low<T>(H, n_b, H.nl_w), H.dion,
-                     (const double*)H.qinv.p, coef, (int)first, P, pb, H.has_s ? y : nullptr, stack,
+                     (const double*)H.qd.p, coef, (int)first, P, pb, H.has_s ? y : nullptr, stack,
                      BR, ress);
   CHS_LAUNCH_CHECK(ctx);
-  // [f C; W_{k+1}] = [0; G] + [M; B M] (f y), or W_{k+1} = G + B (f C)
+  // [f C; W_{k+1}] = [0; G] + [N; B N] (f y), or W_{k+1} = G + B (f C)
   if (H.has_s)
     CHS_TRY(gemm_filter<T>(ctx, 'N', 2 * P, n_b, P, K, 2 * P, y, P, 1.0, stack, 2 * P));
   else
@@ -813,10 +816,13 @@ int chs_bind_projectors(chs_context* ctx, int n_proj, const double* d_beta, cons
   CHS_TRY(tri_inv(ctx, A, Li, P));
   CHS_TRY(zgemm(ctx, 'C', 'N', P, P, P, mk(1.0, 0.0), Li, P, Li, P, mk(0.0, 0.0),
                 (z64*)H.sinv_m.p, P));
-  CHS_TRY(ensure(ctx, H.qinv, (size_t)P * sizeof(double)));
-  hipLaunchKernelGGL(k_stack_m, dim3(ceil_div(pp, 256)), dim3(256), 0, ctx->stream,
-                     (const z64*)H.sinv_m.p, d_q, P, (z64*)H.kstack.p, (double*)H.qinv.p);
+  CHS_TRY(ensure(ctx, H.qd, (size_t)P * sizeof(double)));
+  z64* K = (z64*)H.kstack.p;
+  hipLaunchKernelGGL(k_stack_n, dim3(ceil_div(pp, 256)), dim3(256), 0, ctx->stream,
+                     (const z64*)H.sinv_m.p, d_q, P, K, (double*)H.qd.p);
   CHS_LAUNCH_CHECK(ctx);
+  CHS_TRY(zgemm(ctx, 'N', 'N', P, P, P, mk(1.0, 0.0), (const z64*)H.bmat.p, P, K, 2 * P,
+                mk(0.0, 0.0), K + P, 2 * P));
   H.has_s = true;
   CHS_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return CHS_OK;
