@@ -765,6 +765,7 @@ static int gemm_launch(chs_context* ctx, int choice, int oa, int ob, int m, int 
   const int target = kSplitTargets[(choice >> 4) % kNumSplitTargets];
   // the offset-addressed kernels (3, 4, 5) only while their offsets fit 32 bits;
   // otherwise the bounds-tested kernel of the same tile
+  if (variant > 8) variant = 0;  // no such kernel (CHS_GEMM_CHOICE, a hand-written cache line)
   if (variant == 6 && (oa == 1 || ob != 0 || tri)) variant = 3;
   if (variant >= 7 && (sizeof(T) == 8 || oa == 1 || ob != 0 || tri)) variant = 3;
   if (variant >= 3 && variant != 6) {
