@@ -475,10 +475,15 @@ __global__ void __launch_bounds__(256) k_lanczos_coef(int P, const z64* __restri
 }
 
 // One-workgroup forms of the Lanczos vector steps for blocks of up to
-// kOneLanczos plane waves, where a launch costs more than the vectors' bytes.
-// alpha_j = Re<v|u> + sum_p D_p |w_v,p|^2 into ab[2 j].
-constexpr int kOneLanczos = 32768;
+// kOneLanczos plane waves, where a launch costs more than the vectors' bytes; a
+// lone workgroup streams at a single CU's rate, so longer vectors take the
+// many-workgroup steps. Ten-step bound, one workgroup against many: 2,945 plane
+// waves and 32 projectors 0.49 against 0.56 ms, 9,315 and 256 0.78 against 0.86,
+// 13,133 and 256 0.87 against 0.85, 23,847 and 256 1.22 against 0.98, 23,847
+// without projectors 0.63 against 0.49.
+constexpr int kOneLanczos = 12288;
 
+// alpha_j = Re<v|u> + sum_p D_p |w_v,p|^2 into ab[2 j].
 __global__ void __launch_bounds__(kOneBlock) k_lanczos_alpha(const z64* __restrict__ v,
                                                              const z64* __restrict__ u, int n,
                                                              int P, const double* __restrict__ d,
