@@ -27,6 +27,7 @@
 
 #include "fft.hpp"
 #include "impl.hpp"
+#include "plane_shape.hpp"
 #include "scf_dev.hpp"
 
 namespace chs {
@@ -172,7 +173,7 @@ __global__ void __launch_bounds__(TPB) k_plane(cplx<T>* __restrict__ sbuf, Stick
   // 512 bands: 4.99 ms with, 4.95 without).
   constexpr bool PF = sizeof(T) == 4 && TPB <= 512;
   RowV<N, T> vv;
-  if (PF && rows) vv.load(vz + (PR ? W::row(g) : g) * N, lane);
+  if (PF && rows && g < N) vv.load(vz + (PR ? W::row(g) : g) * N, lane);
   if constexpr (PR)
     zero_window_plane<N, T>(cmp);
   else
@@ -564,26 +565,13 @@ static int plane_launch(chs_context* ctx, int n, const StickArgs& sa, size_t csz
                         size_t extra_bytes = 0) {
   const size_t cmp_bytes = (size_t)n * sa.rs * csz;
   const int lim = max_lds_per_block(ctx);
-  if (cmp_bytes + row_bytes + (size_t)n * sizeof(int32_t) + extra_bytes > (size_t)lim)
-    return set_error(ctx, CHS_ERR_FFT, "plane of %d^3 grid does not fit in LDS (%zu > %d bytes)",
-                     n, cmp_bytes + row_bytes + extra_bytes, lim);
   const int groups = (threads / 64) * (64 / n2);
   const size_t tab_bytes = (size_t)n * sizeof(int32_t) + extra_bytes;  // act_of (+ twiddles)
-  int nrb = (int)((lim - cmp_bytes - tab_bytes) / row_bytes);
-  nrb = std::max(1, std::min(nrb, groups) / std::max(1, nrb_div));
-  // no more row buffers than rows: group g < nrb starts on row g (the plane
-  // kernel loads that row's V_eff ahead of its loop), and a 512-thread
-  // workgroup has more groups than a 32- or 36-point plane has rows
-  nrb = std::min(nrb, n);
-  // the fewest that keep the rounds over the rows and over the active columns,
-  // where that lets another workgroup onto the CU (complex64 at 72 points, 512
-  // threads: 36 of 56 groups, three workgroups in place of two, 0.191 -> 0.174
-  // ms for 160 bands); otherwise whole wavefronts of groups are better
-  // (complex128 at 72 points: 24 in place of 28 groups cost 4%)
-  const int rr = (n + nrb - 1) / nrb, ry = (sa.n_act + nrb - 1) / nrb;
-  const int few = std::max((n + rr - 1) / rr, (sa.n_act + ry - 1) / ry);
-  auto per_cu = [&](int g) { return lim / (int)(cmp_bytes + (size_t)g * row_bytes + tab_bytes); };
-  if (per_cu(few) > per_cu(nrb)) nrb = few;
+  const int nrb =
+      plane_row_buffers(lim, cmp_bytes, row_bytes, tab_bytes, n, sa.n_act, groups, nrb_div);
+  if (nrb == 0)
+    return set_error(ctx, CHS_ERR_FFT, "plane of %d^3 grid does not fit in LDS (%zu > %d bytes)",
+                     n, cmp_bytes + row_bytes + extra_bytes, lim);
   out->nrb = nrb;
   out->threads = threads;
   out->lds = cmp_bytes + (size_t)nrb * row_bytes + tab_bytes;

@@ -1,6 +1,7 @@
 """Plane kernel on grids with fewer rows than a large workgroup has lane
-groups (16 to 36 points): every launch shape the tuner times must stay inside
-V_eff, and H|psi> must be that of a plain numpy transform."""
+groups (16 to 36 points): after the tuner has run every launch shape, H|psi> must
+be that of a plain numpy transform. (That no shape reads V_eff past its end is
+checked on the CPU, in test_plane_shape.py.)"""
 import numpy as np
 import pytest
 
