@@ -568,7 +568,7 @@ static int plane_launch(chs_context* ctx, int n, const StickArgs& sa, size_t csz
   const int groups = (threads / 64) * (64 / n2);
   const size_t tab_bytes = (size_t)n * sizeof(int32_t) + extra_bytes;  // act_of (+ twiddles)
   const int nrb =
-      plane_row_buffers(lim, cmp_bytes, row_bytes, tab_bytes, n, sa.n_act, groups, nrb_div);
+      plane_row_buffers(lim, cmp_bytes, row_bytes, tab_bytes, csz, n, sa.n_act, groups, nrb_div);
   if (nrb == 0)
     return set_error(ctx, CHS_ERR_FFT, "plane of %d^3 grid does not fit in LDS (%zu > %d bytes)",
                      n, cmp_bytes + row_bytes + extra_bytes, lim);

@@ -20,13 +20,13 @@ def row_buffers(tmp_path_factory):
     d = tmp_path_factory.mktemp("shape")
     src = d / "shape.cpp"
     src.write_text('#include "plane_shape.hpp"\nextern "C" int f(size_t l, size_t c, size_t r, '
-                   'size_t t, int n, int na, int g, int d) {\n'
-                   '  return chs::plane_row_buffers(l, c, r, t, n, na, g, d);\n}\n')
+                   'size_t t, size_t z, int n, int na, int g, int d) {\n'
+                   '  return chs::plane_row_buffers(l, c, r, t, z, n, na, g, d);\n}\n')
     so = d / "shape.so"
     subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, str(src), "-o", str(so)],
                    check=True)
     f = ctypes.CDLL(str(so)).f
-    f.argtypes = [ctypes.c_size_t] * 4 + [ctypes.c_int] * 4
+    f.argtypes = [ctypes.c_size_t] * 5 + [ctypes.c_int] * 4
     return f
 
 
@@ -46,7 +46,7 @@ def test_row_buffers_stay_on_the_plane(row_buffers):
         for rs in (n // 2 + 1, n):
             cmp_bytes, row, tab = n * rs * csz, 8 * slots, 4 * n + extra
             groups = threads // 64 * (64 // n2)
-            nrb = row_buffers(LDS, cmp_bytes, row, tab, n, n_act, groups, div)
+            nrb = row_buffers(LDS, cmp_bytes, row, tab, csz, n, n_act, groups, div)
             at = (n, csz, threads, div, n_act, extra, rs, nrb)
             if cmp_bytes + row + tab > LDS:
                 assert nrb == 0, at
@@ -54,9 +54,11 @@ def test_row_buffers_stay_on_the_plane(row_buffers):
             assert 1 <= nrb <= min(n, groups), at  # group g loads row g's V_eff
             assert cmp_bytes + nrb * row + tab <= LDS, at
             some += 1
+            if csz == 16:  # every group that the divisor and the LDS leave
+                assert nrb == min(n, max(1, min(groups, (LDS - cmp_bytes - tab) // row) // div)), at
     assert some > 1000
 
 
 def test_plane_that_does_not_fit(row_buffers):
-    assert row_buffers(LDS, LDS - 100, 101, 0, 64, 30, 28, 1) == 0
-    assert row_buffers(LDS, LDS - 100, 100, 0, 64, 30, 28, 1) == 1
+    assert row_buffers(LDS, LDS - 100, 101, 0, 8, 64, 30, 28, 1) == 0
+    assert row_buffers(LDS, LDS - 100, 100, 0, 8, 64, 30, 28, 1) == 1
