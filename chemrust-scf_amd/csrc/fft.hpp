@@ -489,7 +489,8 @@ template <int N, typename T> struct RowPlanLoad {
 // wavefront per SIMD; 8-byte slots 59). The radix-12 and radix-16 second
 // stages (48, 96, 128 and 144 points) keep whole complex128 values: split, the
 // compiler orders their codelets' sums differently in the last bit, and the
-// eigenvectors Rayleigh-Ritz makes of H|psi> may then change sign.
+// eigenvectors that Rayleigh-Ritz makes of H|psi>, whose signs are those of
+// rounding errors, would differ from those of earlier builds.
 template <int N, typename T> struct Slot {
   static constexpr bool WHOLE = sizeof(T) == 4 || Split<N>::N2 > 9;
   using type = std::conditional_t<WHOLE, cplx<T>, T>;
@@ -527,22 +528,18 @@ template <int N, typename T> struct RowScratch {
   static_assert(STRIDE >= SPAN && PA >= N2 && PB >= N1, "tile layout");
 };
 
-// The 3 x 3 tail's exchange through the group scratch (Mid9Tail): lane
-// (t, x) hands y[c] to lane (t, c). Ends with every read issued.
+// The 3 x 3 tail's exchange through the group scratch (Mid9Tail, complex64:
+// whole values): lane (t, x) hands y[c] to lane (t, c). Ends with every read
+// issued.
 template <int N, int E, typename T>
 __device__ __forceinline__ void tail_exchange(slot_t<N, T>* sc, cplx<T>* y, int t, int j) {
   using MT = Mid9Tail<N, T>;
-  using SL = Slot<N, T>;
-  const cplx<T> v[3] = {y[0], y[1], y[2]};
+  static_assert(Slot<N, T>::WHOLE, "the tail moves whole values");
 #pragma unroll
-  for (int h = 0; h < SL::H; ++h) {
-    if (h) wave_sync();
+  for (int c = 0; c < 3; ++c) sc[E + MT::at(t, j, c)] = y[c];
+  wave_sync();
 #pragma unroll
-    for (int c = 0; c < 3; ++c) sc[E + MT::at(t, j, c)] = SL::put(v[c], h);
-    wave_sync();
-#pragma unroll
-    for (int c = 0; c < 3; ++c) SL::get(y[c], sc[E + MT::at(t, c, j)], h);
-  }
+  for (int c = 0; c < 3; ++c) y[c] = sc[E + MT::at(t, c, j)];
 }
 
 // One line of a plane (element j at line[j ES], ES compile-time) by the N2
@@ -566,8 +563,8 @@ __device__ __forceinline__ void group_fft_line_x(cplx<T>* line, slot_t<N, T>* sc
   Dft<N1, S, T>::run(a);
 #pragma unroll
   for (int k1 = 1; k1 < N1; ++k1) a[k1] = a[k1] * twiddle<S>(tw, lane * k1);
-  // complex128 reads every round's rows (and the tail's) pass by pass, since
-  // its second pass overwrites the tile; complex64 reads them as it goes
+  // split complex128 reads every round's rows pass by pass, since its second
+  // pass overwrites the tile; whole values (and the tail) are read as it goes
   cplx<T> b[MT::RR][N2], y[3];
   const int t = lane / 3, j = lane - 3 * t;
 #pragma unroll
@@ -583,10 +580,6 @@ __device__ __forceinline__ void group_fft_line_x(cplx<T>* line, slot_t<N, T>* sc
 #pragma unroll
           for (int n2 = 0; n2 < N2; ++n2) SL::get(b[r][n2], sc[(lane + r * N2) * PA + n2], h);
         }
-      if constexpr (MT::on) {
-#pragma unroll
-        for (int q = 0; q < 3; ++q) SL::get(y[q], sc[(N2 + t) * PA + 3 * q + j], h);
-      }
     }
   }
 #pragma unroll
@@ -605,10 +598,8 @@ __device__ __forceinline__ void group_fft_line_x(cplx<T>* line, slot_t<N, T>* sc
   }
   if constexpr (MT::on) {  // rows k1 = 9 + t by lanes 3 t + j (Mid9Tail)
     const int k1 = N2 + t;
-    if constexpr (SL::H == 1) {
 #pragma unroll
-      for (int q = 0; q < 3; ++q) SL::get(y[q], sc[k1 * PA + 3 * q + j], 0);
-    }
+    for (int q = 0; q < 3; ++q) y[q] = sc[k1 * PA + 3 * q + j];
     Dft<3, S, T>::run(y);
     y[1] = y[1] * twiddle<S>(tw, (N / 9) * j);
     y[2] = y[2] * twiddle<S>(tw, (N / 9) * 2 * j);
@@ -687,7 +678,7 @@ __device__ __forceinline__ void row_apply_v(cplx<T>* crow, slot_t<N, T>* sc, con
     Dft<N1, 1, T>::run(a);
 #pragma unroll
     for (int k1 = 1; k1 < N1; ++k1) a[k1] = a[k1] * rp.w1(k1);
-    // (complex128: both passes' reads here, as in group_fft_line_x)
+    // (split complex128: both passes' reads here, as in group_fft_line_x)
 #pragma unroll
     for (int h = 0; h < SL::H; ++h) {
       if (h) wave_sync();
@@ -701,10 +692,6 @@ __device__ __forceinline__ void row_apply_v(cplx<T>* crow, slot_t<N, T>* sc, con
 #pragma unroll
             for (int n2 = 0; n2 < N2; ++n2) SL::get(b[r][n2], sc[(lane + r * N2) * PA + n2], h);
           }
-        if constexpr (MT::on) {
-#pragma unroll
-          for (int q = 0; q < 3; ++q) SL::get(y[q], sc[tk1 * PA + 3 * q + tj], h);
-        }
       }
     }
   }
@@ -732,10 +719,8 @@ __device__ __forceinline__ void row_apply_v(cplx<T>* crow, slot_t<N, T>* sc, con
     }
   }
   if constexpr (MT::on) {
-    if constexpr (SL::H == 1) {
 #pragma unroll
-      for (int q = 0; q < 3; ++q) SL::get(y[q], sc[tk1 * PA + 3 * q + tj], 0);
-    }
+    for (int q = 0; q < 3; ++q) y[q] = sc[tk1 * PA + 3 * q + tj];
     Dft<3, 1, T>::run(y);
     y[1] = y[1] * rp.w9(1);
     y[2] = y[2] * rp.w9(2);
@@ -775,7 +760,7 @@ __device__ __forceinline__ void row_apply_v(cplx<T>* crow, slot_t<N, T>* sc, con
     }
     if constexpr (MT::on) {
 #pragma unroll
-      for (int q = 0; q < 3; ++q) sc[(tj + 3 * q) * PB + tk1] = SL::put(y[q], h);
+      for (int q = 0; q < 3; ++q) sc[(tj + 3 * q) * PB + tk1] = y[q];
     }
     if constexpr (PF)
       if (h == SL::H - 1 && next_vrow) vv.load(next_vrow, lane);
