@@ -206,6 +206,14 @@ __attribute__((amdgpu_waves_per_eu(MfmaTile<T, V>::WAVES))) k_gemm_mfma(int m, i
   int bm, bn, bz;
   if (!gemm_block((m + BM - 1) / BM, (n + BN - 1) / BN, ksplit, nfast, &bm, &bn, &bz)) return;
   if (tri && bm * BM >= (bn + 1) * BN) return;  // Hermitian product: tiles below the diagonal
+  // Workgroups that share a CU (every 256th or so) get two wave priorities, so
+  // that their product phases do not run in step and leave the matrix cores
+  // idle together. Complex64, without and with: 80,725 x 512 x 864 1.825 and
+  // 1.785 ms, 63,077 x 360 x 864 1.094 and 1.073, 80,725 x 512 x 512 1.122 and
+  // 1.088; short sums lose by it (17,071 x 192 x 256 69.7 and 72.0 us), as do
+  // the 96-row tiles, three wavefronts per SIMD
+  if constexpr (sizeof(T) == 4 && V == 1 && CL)
+    if (klen >= 512 && ((blockIdx.x >> 8) & 1)) __builtin_amdgcn_s_setprio(2);
   constexpr int NA = BM * BK / 256, NB = BN * BK / 256;  // staged elements per thread
   // one padding element per row: the K-major (transposing) stores of T / C
   // operands then hit distinct banks across each phase of lanes, while the
@@ -309,12 +317,6 @@ __attribute__((amdgpu_waves_per_eu(MfmaTile<T, V>::WAVES))) k_gemm_mfma(int m, i
       Bs[kk][c] = rb[j];
     }
   };
-  // Workgroups that share a CU (every 256th or so) get two wave priorities, so
-  // that their product phases do not run in step and leave the matrix cores
-  // idle together (80,725 x 512 x 864 complex64: 1.83 -> 1.79 ms; the 96-row
-  // tiles, three wavefronts per SIMD, lose by it)
-  if constexpr (sizeof(T) == 4 && V == 1 && CL)
-    if ((blockIdx.x >> 8) & 1) __builtin_amdgcn_s_setprio(2);
   auto products = [&]() {
 #pragma unroll
     for (int s = 0; s < BK / 4; ++s) {
