@@ -118,10 +118,12 @@ constexpr int kMlpBlocks0 = 1024, kMlpBlocks1 = 256;  // 4 (PASS 0) or 1 wavefro
 // h = silu(z), ds = silu'(z) from one sigmoid: 1 / (1 + e^-z) as the hardware
 // reciprocal with one Newton step, and z / (1 + e^-z) from it with a residual
 // step (both round as the division does; without the second step the loss and
-// gradient errors double). The sum is kept finite so that the steps have no
-// inf * 0: below z = -69 the sigmoid is 1e-30.
+// gradient errors double). Below z = -69, where both are under 1e-28, z is taken
+// as -69, so that the sum stays finite and the steps have no inf * 0 (the maximum
+// hands a NaN on).
 __device__ __forceinline__ void silu2(float z, float& h, float& ds) {
-  const float d = fminf(1.0f + expf(-z), 1e30f);
+  z = __builtin_elementwise_maximum(z, -69.0f);
+  const float d = 1.0f + expf(-z);
   float r = __builtin_amdgcn_rcpf(d);
   r = fmaf(fmaf(-d, r, 1.0f), r, r);
   h = z * r;
