@@ -830,9 +830,11 @@ int heev_tridiag(chs_context* ctx, z64* A, int n, double* w, z64* U) {
   hipLaunchKernelGGL(k_tri_to_complex, dim3(ceil_div((size_t)n * n, 256)), dim3(256), 0,
                      ctx->stream, ws.zt, n, U);
   CHS_LAUNCH_CHECK(ctx);
-  // 3. U <- Q U, blocks of reflectors from the last to the first (32-wide
-  // products: 64 x 64 tiles keep one to eight workgroups busy, the small-product
-  // kernel up to 80; 160-band Rayleigh-Ritz 3.00 -> 2.93 ms)
+  // 3. U <- Q U, blocks of reflectors from the last to the first. The four
+  // products of a block are 32 wide or deep: 64 x 64 tiles make 1, 3, 3 and 9
+  // workgroups of them at n = 160 (2, 16, 8 and 64 at 512), the small-product
+  // kernel up to 2, 10, 5 and 25 (4, 64, 16 and 256); 160-band Rayleigh-Ritz
+  // 3.00 -> 2.93 ms
   const z64 one = mk(1.0, 0.0), zero = mk(0.0, 0.0), mone = mk(-1.0, 0.0);
   const int nref = n - 1;
   for (int kb = ((nref - 1) / kWY) * kWY; nref > 0 && kb >= 0; kb -= kWY) {
