@@ -866,26 +866,32 @@ constexpr double kSmallWork = 4e9;
 // Split-K target of a complex128 product, by its shape alone. The order of its
 // sums, hence the last bits of H_sub and S_sub, sets the signs of Rayleigh-Ritz's
 // eigenvectors (inverse iteration keeps the sign of a rounding error), so it must
-// not follow the tuner's timings: candidates 1% apart (864 x 512 x 80,725: 36
-// slices 3.53 ms, 18 slices 3.57 ms) were picked differently from one context to
-// the next. The smallest target with at least kMinSlices slices (kMinSlicesTri
-// where only the upper tiles are computed), as long as slices stay kMinSlice
-// long: fewer leave part of the chip waiting for the last workgroups (512 x 512
-// upper tiles of K = 80,725: 28 slices 1.70 ms, 56 1.57 ms; 864 x 360 x 63,077:
-// 12 slices 2.11 ms, 24 2.07 ms), shorter ones pay for their partial sums (256 x
-// 256 x 20,815: 32 slices 0.162 ms, 62 0.176 ms; 864 x 864 x 864: 2 slices 0.103
-// ms, 4 0.117 ms). Over 60 shapes of the 64- and 216-atom cells it takes the
-// fastest split or one within 1.5%, but for the upper tiles of 257 to 384 bands
-// (up to 5%).
-constexpr int kMinSlices = 24, kMinSlicesTri = 48, kMinSlice = 512;
-
+// not follow the tuner's timings: candidates 1% apart (864 x 512 x 80,725: 18
+// slices 3.42 ms, 36 slices 3.44 ms) were picked differently from one context to
+// the next. The smallest target that gives enough slices, as long as they stay
+// longer than a least length; `ms` below is without and with that target's split.
+//  - All tiles: 17 slices whose workgroups fill the target to 97% (864 x 360 x
+//    63,077: 12 slices 2.11 ms, 24 2.07; 864 x 440 x 60,245: 20 slices fill 96%,
+//    2.32, 41 fill 98%, 2.29), no shorter than 800 (256 x 400 x 23,847: 36 slices
+//    of 672 0.305 ms, 18 of 1,328 0.295).
+//  - Upper tiles only: 48 slices in a multiple of 8 or 70, since the tiles below
+//    the diagonal are launched too and end at once, and with a broken number of
+//    slices an XCD gets more of the others (512 x 512 x 80,725: 28 slices 1.70 ms,
+//    56 1.57; 302 x 302 x 74,509: 68 slices 0.598, 134 0.550), no shorter than 272
+//    (300 x 300 x 13,133: 52 slices of 256 0.141 ms, 33 of 400 0.112).
+// Of 180 shapes of the 64- and 216-atom cells all but nine take the split that was
+// timed fastest or one within 1.5% of it, those one within 5%.
 static int fixed_split_target(int m, int n, int k, bool tri) {
-  int ks, kl, ti = 0;
-  variant_plan<double>(3, m, n, k, kSplitTargets[0], tri, &ks, &kl);
-  while (ks < (tri ? kMinSlicesTri : kMinSlices) && ti + 1 < kNumSplitTargets) {
-    variant_plan<double>(3, m, n, k, kSplitTargets[ti + 1], tri, &ks, &kl);
-    if (kl < kMinSlice) break;
-    ++ti;
+  int bm, bn, bk, ks, kl, ti = 0;
+  tile_dims<double>(3, &bm, &bn, &bk);
+  const double tiles = (double)ceil_div(m, bm) * ceil_div(n, bn);
+  for (int t = 0; t < kNumSplitTargets; ++t) {
+    variant_plan<double>(3, m, n, k, kSplitTargets[t], tri, &ks, &kl);
+    if (t > 0 && kl < (tri ? 272 : 800)) break;
+    ti = t;
+    if (tri ? ks >= 70 || (ks >= 48 && ks % 8 == 0)
+            : ks >= 17 && tiles * ks >= 0.97 * kSplitTargets[t])
+      break;
   }
   return ti;
 }
