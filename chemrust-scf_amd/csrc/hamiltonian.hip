@@ -167,8 +167,8 @@ __global__ void __launch_bounds__(TPB) k_plane(cplx<T>* __restrict__ sbuf, Stick
   // Rows t = g, g + nrb, ... With PF each row's V_eff is loaded during the
   // work before it (the first row's from here on, the others' during the
   // row before); that holds 12 more registers per lane across the row, which
-  // the 256-thread complex64 shape has (two wavefronts per SIMD, 256
-  // registers each), the 512-thread one with the LDS twiddle plan, and the
+  // the 256-thread complex64 shape has (137 at 108 points, three wavefronts per
+  // SIMD), the 512-thread one with the LDS twiddle plan (100, four), and the
   // 1024-thread shape does not. complex128 gains nothing from it (108 points,
   // 512 bands: 4.99 ms with, 4.95 without).
   constexpr bool PF = sizeof(T) == 4 && TPB <= 512;
